@@ -13,7 +13,7 @@
 #include <tuple>
 #include <string>
 #include <vector>
-#include "m2c_kernels.h"
+#include "m2c_stage_u.h"
 #include "m2c_multiphase.h"
 #include "m2c_reinit.h"
 #include "m2c_band.h"
@@ -83,9 +83,14 @@ struct m2cx_solver {
   // interface Riemann problems are solved on stream (fork / join events)
   hipStream_t stream2 = nullptr;
   hipEvent_t ev_fork = nullptr, ev_join = nullptr;
-  unsigned char* tflag = nullptr;
-  long tflag_n = 0;
   bool overlap = false;
+  // stage tiles: tflag marks the mixed ones (k_tile_mixed, once per step);
+  // the others run the one-material kernel when the scheme has one (ustage).
+  // A solver of one material without inactive cells has no mixed tile and
+  // needs no flags, unless its steps are captured (flags_always: the IDs may
+  // be uploaded anew between replays).
+  unsigned char* tflag = nullptr;
+  bool ustage = false, has_inactive = false, flags_always = false;
   // level-set reinitialization
   RBuf rb{};
   double reinit_cfl = 0.8;  // the reinitializer's CFL, lowered by its failsafe
@@ -617,21 +622,24 @@ static int create_impl(const m2cx_grid* grid, const m2cx_material* mats, int nma
     HIPCHK(h, hipMalloc(&lsk, LSKcoef.size() * 4));
     HIPCHK(h, hipMemcpy(lsk, LSKcoef.data(), LSKcoef.size() * 4, hipMemcpyHostToDevice));
     fv.lsk = lsk;
-    // second stream and tile flags for overlapping the stage kernel with the
-    // interface Riemann solve (default priority, like the solver's stream)
+    // second stream for overlapping the stage kernel with the interface
+    // Riemann solve (default priority, like the solver's stream)
     if (!getenv("M2C_NO_OVERLAP")) {
       HIPCHK(h, hipStreamCreateWithFlags(&h->stream2, hipStreamNonBlocking));
       HIPCHK(h, hipEventCreateWithFlags(&h->ev_fork, hipEventDisableTiming));
       HIPCHK(h, hipEventCreateWithFlags(&h->ev_join, hipEventDisableTiming));
-      long mt = 0;
-      for (const TileVariant& t : kTiles)
-        mt = std::max(mt, (long)((NX + t.bx - 1) / t.bx) * ((NY + t.by - 1) / t.by) * ((NZ + t.bz - 1) / t.bz));
-      HIPCHK(h, hipMalloc(&h->tflag, mt));
-      h->tflag_n = mt;
       h->overlap = true;
     }
-    
   }
+  long mt = 0;
+  for (const TileVariant& t : kTiles)
+    mt = std::max(mt, (long)((NX + t.bx - 1) / t.bx) * ((NY + t.by - 1) / t.by) * ((NZ + t.bz - 1) / t.bz));
+  HIPCHK(h, hipMalloc(&h->tflag, mt));
+  // the one-material stage kernel: what its code leaves out (m2c_stage_u.h)
+  h->ustage = s.flux != M2CX_FLUX_GODUNOV && s.rec_type == M2CX_REC_LINEAR && s.var_type == M2CX_VAR_PRIMITIVE;
+  for (size_t q = 0; q < Acoef.size(); q++)
+    h->ustage = h->ustage && Acoef[q] == 1.0 && Bcoef[q] == 1.0 && (s.limiter != M2CX_LIM_VANALBADA || Kcoef[q] == 2);
+  for (int q = 0; q < nmat; q++) h->ustage = h->ustage && eos_in_range(M.m[q]);
   if (h->multimat) fill_iface_ls(h);
   HIPCHK(h, hipStreamSynchronize(h->stream));
   return 0;
@@ -708,7 +716,13 @@ int m2cx_upload(m2cx_solver* h, int field, const void* host) {
   const long n = h->ncells;
   if (field == M2CX_FIELD_ID) {
     HIPCHK(h, hipMemcpyAsync(h->staging_i, host, n * 4, hipMemcpyHostToDevice, h->stream));
-    k_i32_to_u8<<<grid_blocks(n), 256, 0, h->stream>>>(h->staging_i, h->ID, n);
+    k_i32_to_u8<<<grid_blocks(n), 256, 0, h->stream>>>(h->staging_i, h->ID, n, h->s.inactive, &h->cnt->inactive_seen);
+    if (!h->multimat) {
+      int seen = 0;
+      HIPCHK(h, hipMemcpyAsync(&seen, &h->cnt->inactive_seen, sizeof seen, hipMemcpyDeviceToHost, h->stream));
+      HIPCHK(h, hipStreamSynchronize(h->stream));
+      h->has_inactive = seen != 0;
+    }
   } else if (field == M2CX_FIELD_PHI) {
     if (!h->mp.phi) return fail(h, M2CX_E_ARG, "no level set");
     HIPCHK(h, hipMemcpyAsync(h->mp.phi, host, n * 8, hipMemcpyHostToDevice, h->stream));
@@ -782,6 +796,9 @@ int m2cx_get_time(m2cx_solver* h, double* t, double* dt, int* time_step) {
   return 0;
 }
 
+// whether the stage launches of the next step need the tile flags
+static bool needs_tflags(const m2cx_solver* h) { return h->multimat || h->has_inactive || h->flags_always; }
+
 static StageArgs stage_args(m2cx_solver* h, int vin, int vout, int mode) {
   StageArgs a{};
   a.g = h->g;
@@ -799,19 +816,24 @@ static StageArgs stage_args(m2cx_solver* h, int vin, int vout, int mode) {
   a.mode = mode;
   a.cnt = h->cnt;
   a.gflux = h->gflux;
+  a.tflag = needs_tflags(h) ? h->tflag : nullptr;
   return a;
 }
 
 extern "C++" {
 static constexpr int kNumTiles = 4;
 
+// one work-group per tile, padded to a multiple of the XCD count (see
+// xcd_tile for the tile order)
+template <int BX, int BY, int BZ>
+static dim3 stage_grid(const DevGrid& g) {
+  const long ntiles = (long)((g.NX + BX - 1) / BX) * ((g.NY + BY - 1) / BY) * ((g.NZ + BZ - 1) / BZ);
+  return dim3((unsigned)((ntiles + NXCD - 1) / NXCD * NXCD));
+}
+
 template <int BX, int BY, int BZ, bool GEN>
 static void launch_stage_tile(m2cx_solver* h, const StageArgs& a, int mode, hipStream_t st) {
-  // one work-group per tile, padded to a multiple of the XCD count (see
-  // k_stage for the tile order)
-  const long ntiles = (long)((h->g.NX + BX - 1) / BX) * ((h->g.NY + BY - 1) / BY) * ((h->g.NZ + BZ - 1) / BZ);
-  const long per = (ntiles + NXCD - 1) / NXCD;
-  const dim3 grid((unsigned)(per * NXCD));
+  const dim3 grid = stage_grid<BX, BY, BZ>(h->g);
   constexpr int nt = BX * BY * BZ;
   switch (mode) {
     case MODE_RESIDUAL: k_stage<MODE_RESIDUAL, BX, BY, BZ, GEN><<<grid, nt, 0, st>>>(a); break;
@@ -823,11 +845,33 @@ static void launch_stage_tile(m2cx_solver* h, const StageArgs& a, int mode, hipS
   }
 }
 
+template <int BX, int BY, int BZ>
+static void launch_ustage_tile(m2cx_solver* h, const StageArgs& a, int mode, hipStream_t st) {
+  const dim3 grid = stage_grid<BX, BY, BZ>(h->g);
+  constexpr int nt = BX * BY * BZ;
+  switch (mode) {
+    case MODE_RESIDUAL: k_stage_u<MODE_RESIDUAL, BX, BY, BZ><<<grid, nt, 0, st>>>(a); break;
+    case MODE_STAGE1: k_stage_u<MODE_STAGE1, BX, BY, BZ><<<grid, nt, 0, st>>>(a); break;
+    case MODE_RK2_FINAL: k_stage_u<MODE_RK2_FINAL, BX, BY, BZ><<<grid, nt, 0, st>>>(a); break;
+    case MODE_RK3_STAGE2: k_stage_u<MODE_RK3_STAGE2, BX, BY, BZ><<<grid, nt, 0, st>>>(a); break;
+    case MODE_RK3_FINAL: k_stage_u<MODE_RK3_FINAL, BX, BY, BZ><<<grid, nt, 0, st>>>(a); break;
+    case MODE_FE: k_stage_u<MODE_FE, BX, BY, BZ><<<grid, nt, 0, st>>>(a); break;
+  }
+}
+
+static void launch_ustage_variant(m2cx_solver* h, const StageArgs& a, int mode, int v, hipStream_t st) {
+  switch (v) {
+    case 1: launch_ustage_tile<32, 4, 2>(h, a, mode, st); break;
+    case 2: launch_ustage_tile<8, 8, 4>(h, a, mode, st); break;
+    case 3: launch_ustage_tile<16, 8, 2>(h, a, mode, st); break;
+    default: launch_ustage_tile<16, 4, 4>(h, a, mode, st); break;
+  }
+}
+
 // Reconstruction in conservative or characteristic variables runs one tile
 // shape (16x4x4) of the general kernel; primitive variables choose the tuned
 // tile of the primitive-only kernel.
-static void launch_stage_variant(m2cx_solver* h, const StageArgs& a, int mode, int v, hipStream_t st = nullptr) {
-  if (!st) st = h->stream;
+static void launch_stage_variant(m2cx_solver* h, const StageArgs& a, int mode, int v, hipStream_t st) {
   if (a.s.var_type != M2CX_VAR_PRIMITIVE && a.s.rec_type == M2CX_REC_LINEAR) {
     launch_stage_tile<16, 4, 4, true>(h, a, mode, st);
     return;
@@ -850,19 +894,29 @@ static void stage_tile_dims(const m2cx_solver* h, int& tx, int& ty, int& tz) {
   tx = t.bx; ty = t.by; tz = t.bz;
 }
 
-// phase 0: all tiles on the solver's stream; 1: tiles without interface
-// faces on stream2 (timed as "stage"); 2: the others on the solver's stream
-// (timed as "stage_if")
+// phase 0: all tiles on the solver's stream; 1: the tiles of one material on
+// stream2 (timed as "stage"); 2: the mixed ones on the solver's stream (timed
+// as "stage_if")
 static void launch_stage(m2cx_solver* h, int vin, int vout, int mode, int phase = 0) {
   StageArgs a = stage_args(h, vin, vout, mode);
-  a.phase = phase;
-  a.tflag = h->tflag;
   hipStream_t st = (phase == 1) ? h->stream2 : h->stream;
   const char* name = (phase == 2) ? "stage_if" : "stage";
+  const int v = h->tile < 0 ? 0 : h->tile;
   hipEvent_t e0{};
   tic(h, name, &e0, st);
-  launch_stage_variant(h, a, mode, h->tile < 0 ? 0 : h->tile, st);
+  if (h->ustage && phase != 2) launch_ustage_variant(h, a, mode, v, st);
+  a.phase = (h->ustage && phase == 0) ? 2 : phase;
+  if (!h->ustage || phase == 2 || (phase == 0 && a.tflag)) launch_stage_variant(h, a, mode, v, st);
   toc(h, name, e0, st);
+}
+
+// Marks the mixed stage tiles, after the step's interface list is built (IDs
+// do not change between stages).
+static void tile_flags(m2cx_solver* h) {
+  int tx, ty, tz;
+  stage_tile_dims(h, tx, ty, tz);
+  const int nt = ((h->g.NX + tx - 1) / tx) * ((h->g.NY + ty - 1) / ty) * ((h->g.NZ + tz - 1) / tz);
+  k_tile_mixed<<<(nt + 3) / 4, 256, 0, h->stream>>>(h->g, h->s.inactive, h->ID, h->tflag, tx, ty, tz, nt);
 }
 
 // Tile-shape autotuner: times the residual launch of every variant on the
@@ -893,16 +947,17 @@ static int autotune(m2cx_solver* h, float* ms_out) {
   }
   int err0 = 0;
   HIPCHK(h, hipMemcpy(&err0, &h->cnt->error, sizeof(int), hipMemcpyDeviceToHost));
-  StageArgs a = stage_args(h, 0, -1, MODE_RESIDUAL);
   hipEvent_t e0, e1;
   HIPCHK(h, hipEventCreate(&e0));
   HIPCHK(h, hipEventCreate(&e1));
   int best = 0;
   float best_ms = 1e30f;
   for (int v = 0; v < kNumTiles; v++) {
-    launch_stage_variant(h, a, MODE_RESIDUAL, v);  // warm
+    h->tile = v;
+    if (needs_tflags(h)) tile_flags(h);
+    launch_stage(h, 0, -1, MODE_RESIDUAL);  // warm
     HIPCHK(h, hipEventRecord(e0, h->stream));
-    for (int r = 0; r < 3; r++) launch_stage_variant(h, a, MODE_RESIDUAL, v);
+    for (int r = 0; r < 3; r++) launch_stage(h, 0, -1, MODE_RESIDUAL);
     HIPCHK(h, hipEventRecord(e1, h->stream));
     HIPCHK(h, hipEventSynchronize(e1));
     float ms = 0;
@@ -1015,6 +1070,7 @@ int m2cx_compute_residual(m2cx_solver* h, int v_field, int capture_riemann) {
   HIPCHK(h, hipSetDevice(h->device));
   if (int rc = ensure_slab(h)) return rc;
   if (h->multimat) mp_classify(h->mp, h->g, h->s, h->ID, h->cnt, h->stream);
+  if (needs_tflags(h)) tile_flags(h);
   interface_stage(h, v_field, capture_riemann);
   launch_stage(h, v_field, -1, MODE_RESIDUAL);
   HIPCHK(h, hipGetLastError());
@@ -1518,16 +1574,6 @@ static void split_stage(m2cx_solver* h, const StageSpec& sp) {
   if (sp.ls_which >= 0) levelset_stage(h, sp.vin, sp.ls_which);
 }
 
-// marks the stage-kernel tiles that hold a cell of an interface face (after
-// the step's interface list is built)
-static void tile_flags(m2cx_solver* h) {
-  int tx, ty, tz;
-  stage_tile_dims(h, tx, ty, tz);
-  const long nt = (long)((h->g.NX + tx - 1) / tx) * ((h->g.NY + ty - 1) / ty) * ((h->g.NZ + tz - 1) / tz);
-  k_clear_u8<<<blocks_for(nt), 256, 0, h->stream>>>(h->tflag, nt);
-  k_tile_flags<<<blocks_for(h->mp.L.cap), 256, 0, h->stream>>>(h->g, h->mp.L, h->cnt, h->tflag, tx, ty, tz);
-}
-
 // One TimeIntegrator step with dt already in cnt->dt (TimeIntegrator.cpp:167-715)
 static int step_kernels(m2cx_solver* h) {
   const int ti = h->sch.integrator;
@@ -1546,7 +1592,7 @@ static int step_kernels(m2cx_solver* h) {
     swap_ls(h, q);
     if (unbuilt) return fail(h, M2CX_E_ARG, "the narrow band of the level set has not been constructed");
   }
-  if (h->overlap) tile_flags(h);
+  if (needs_tflags(h)) tile_flags(h);
   if (ti == M2CX_TI_FORWARD_EULER && h->overlap) {
     split_stage(h, StageSpec{0, 1, MODE_FE, 1, 0, -1});
     for (int p = 0; p < 5; p++) std::swap(h->V[0][p], h->V[1][p]);
@@ -2074,6 +2120,7 @@ struct m2cx_ensemble {
   // and tile-count prefix sums
   struct StageClass {
     int v = 0;                 // tile variant (kTiles index)
+    bool ustage = false;       // one-material tiles run k_stage_u_multi
     std::vector<m2cx_solver*> members;
     StageArgs* tab[3][2] = {};
     int* toff = nullptr;
@@ -2103,8 +2150,8 @@ static bool ens_riemann_member(const m2cx_solver* h) {
 }
 
 extern "C++" {
-// k_stage_multi for one class, stage and phase (1: tiles without interface
-// faces, 2: the others) on stream `st`
+// k_stage_multi (k_stage_u_multi) for one class, stage and phase (1: tiles of
+// one material, 2: the mixed ones) on stream `st`
 template <int BX, int BY, int BZ>
 static void launch_class_tile(const m2cx_ensemble::StageClass& c, const StageArgs* tab, int mode, hipStream_t st) {
   const long per = ((long)c.ntiles + NXCD - 1) / NXCD;
@@ -2118,9 +2165,31 @@ static void launch_class_tile(const m2cx_ensemble::StageClass& c, const StageArg
     case MODE_RK3_FINAL: k_stage_multi<MODE_RK3_FINAL, BX, BY, BZ><<<grid, nt, 0, st>>>(tab, c.toff, nm); break;
   }
 }
+template <int BX, int BY, int BZ>
+static void launch_class_utile(const m2cx_ensemble::StageClass& c, const StageArgs* tab, int mode, hipStream_t st) {
+  const long per = ((long)c.ntiles + NXCD - 1) / NXCD;
+  const dim3 grid((unsigned)(per * NXCD));
+  const int nm = (int)c.members.size();
+  constexpr int nt = BX * BY * BZ;
+  switch (mode) {
+    case MODE_STAGE1: k_stage_u_multi<MODE_STAGE1, BX, BY, BZ><<<grid, nt, 0, st>>>(tab, c.toff, nm); break;
+    case MODE_RK2_FINAL: k_stage_u_multi<MODE_RK2_FINAL, BX, BY, BZ><<<grid, nt, 0, st>>>(tab, c.toff, nm); break;
+    case MODE_RK3_STAGE2: k_stage_u_multi<MODE_RK3_STAGE2, BX, BY, BZ><<<grid, nt, 0, st>>>(tab, c.toff, nm); break;
+    case MODE_RK3_FINAL: k_stage_u_multi<MODE_RK3_FINAL, BX, BY, BZ><<<grid, nt, 0, st>>>(tab, c.toff, nm); break;
+  }
+}
 
 static void launch_class(const m2cx_ensemble::StageClass& c, int q, int phase, int mode, hipStream_t st) {
   const StageArgs* tab = c.tab[q][phase - 1];
+  if (c.ustage && phase == 1) {
+    switch (c.v) {
+      case 1: launch_class_utile<32, 4, 2>(c, tab, mode, st); break;
+      case 2: launch_class_utile<8, 8, 4>(c, tab, mode, st); break;
+      case 3: launch_class_utile<16, 8, 2>(c, tab, mode, st); break;
+      default: launch_class_utile<16, 4, 4>(c, tab, mode, st); break;
+    }
+    return;
+  }
   switch (c.v) {
     case 1: launch_class_tile<32, 4, 2>(c, tab, mode, st); break;
     case 2: launch_class_tile<8, 8, 4>(c, tab, mode, st); break;
@@ -2154,9 +2223,7 @@ static void ensemble_step(m2cx_ensemble* e) {
   stage_specs(e->ti, sp);
   // split: the member's stage launch is divided by tiles as in split_stage
   auto split = [e](const m2cx_solver* h) { return e->overlap && ens_riemann_member(h); };
-  if (e->overlap)
-    for (m2cx_solver* h : act)
-      if (split(h)) tile_flags(h);
+  for (m2cx_solver* h : act) tile_flags(h);
   for (int q = 0; q < e->nstages; q++) {
     for (m2cx_solver* h : act) {
       recon_stage(h, sp[q].vin);
@@ -2209,6 +2276,7 @@ struct EnsembleStreamSwap {
   std::vector<hipStream_t> s2;
   explicit EnsembleStreamSwap(m2cx_ensemble* e_) : e(e_), s2(e_->m.size()) {
     for (size_t i = 0; i < e->m.size(); i++) {
+      e->m[i]->flags_always = true;
       e->m[i]->stream = e->stream;
       s2[i] = e->m[i]->stream2;
       e->m[i]->stream2 = e->stream2;
@@ -2216,6 +2284,7 @@ struct EnsembleStreamSwap {
   }
   ~EnsembleStreamSwap() {
     for (size_t i = 0; i < e->m.size(); i++) {
+      e->m[i]->flags_always = false;
       e->m[i]->stream = e->m[i]->stream_saved;
       e->m[i]->stream2 = s2[i];
     }
@@ -2252,13 +2321,15 @@ static int ensemble_build(m2cx_ensemble* e) {
   free_classes(e);
   e->classed.clear();
   if (e->overlap) {
-    std::map<int, m2cx_ensemble::StageClass> bytile;
+    std::map<std::pair<int, bool>, m2cx_ensemble::StageClass> bytile;
     for (size_t i = 0; i < e->m.size(); i++) {
       m2cx_solver* h = e->m[i];
       if (!e->active[i] || !ens_riemann_member(h)) continue;
       if (h->s.var_type != M2CX_VAR_PRIMITIVE && h->s.rec_type == M2CX_REC_LINEAR) continue;
-      auto& c = bytile[h->tile < 0 ? 0 : h->tile];
-      c.v = h->tile < 0 ? 0 : h->tile;
+      const int v = h->tile < 0 ? 0 : h->tile;
+      auto& c = bytile[{v, h->ustage}];
+      c.v = v;
+      c.ustage = h->ustage;
       c.members.push_back(h);
     }
     for (auto& kv : bytile) {
@@ -2281,7 +2352,6 @@ static int ensemble_build(m2cx_ensemble* e) {
           for (m2cx_solver* h : cc.members) {
             StageArgs a = stage_args(h, sp[q].vin, sp[q].vout, sp[q].mode);
             a.phase = phase;
-            a.tflag = h->tflag;
             tab.push_back(a);
           }
           EHIPCHK(e, hipMalloc(&cc.tab[q][phase - 1], tab.size() * sizeof(StageArgs)));
@@ -2489,6 +2559,8 @@ int m2cx_initialize(m2cx_solver* h, const double* default_state, int default_id,
                                                         h->sch.ls_materialid, diag);
   // boundary fill: state, ghost IDs, level set (ApplyBoundaryConditions,
   // UpdateMaterialIDAtGhostNodes, LevelSetOperator::ApplyBoundaryConditions)
+  if (default_id == h->s.inactive) h->has_inactive = true;
+  for (const InitGeom& b : G) h->has_inactive = h->has_inactive || b.id == h->s.inactive;
   k_apply_bc<<<grid_blocks(nin), 256, 0, h->stream>>>(h->g, f5(h, h->V[0]));
   const long nf = 2L * ((long)h->g.NY * h->g.NZ + (long)h->g.NX * h->g.NZ + (long)h->g.NX * h->g.NY);
   k_ghost_ids<<<grid_blocks(nf), 256, 0, h->stream>>>(h->g, h->ID);

@@ -21,6 +21,8 @@ struct DevCounters {
   double t, dt, cfl, dts, tmax;
   int time_step, pad2;
   unsigned long long unresolved_total;  // cells left unresolved by the state update, summed
+  int inactive_seen;  // an uploaded ID field held the inactive material
+  int pad3;
 };
 
 enum StageMode { MODE_RESIDUAL = 0, MODE_STAGE1 = 1, MODE_RK2_FINAL = 2, MODE_RK3_STAGE2 = 3, MODE_RK3_FINAL = 4,
@@ -56,8 +58,8 @@ struct StageArgs {
   const int* fidx[3];
   IfaceList L;
   int mode;
-  // 0: every tile; 1: only tiles without interface faces; 2: only tiles with
-  // them (tflag per tile, set by k_tile_flags for this tile shape)
+  // 0: every tile; 1: only tiles of one material; 2: only mixed ones (tflag
+  // per tile, set by k_tile_mixed for this tile shape)
   int phase;
   const unsigned char* tflag;
   DevCounters* cnt;
@@ -153,6 +155,55 @@ struct TileShape {
 // with equal tables share a slot; Scheme::mset selects it).
 constexpr int MAX_MAT_SETS = 32;
 __constant__ DevMats c_mats[MAX_MAT_SETS];
+
+// What a cell does with its residual r: store it, or the Runge-Kutta
+// combination of the stage, conversion to primitive variables, clipping and
+// the boundary fill of the new state.
+template <int MODE>
+__device__ __forceinline__ void stage_update(const StageArgs& a, const DevEos& E, int i, int j, int k, long c,
+                                             const double* r) {
+  if (MODE == MODE_RESIDUAL) {
+    store5(a.R, c, r);
+    return;
+  }
+  const double dt = a.cnt->dt;
+  double u[5], v[5];
+  if (MODE == MODE_STAGE1 || MODE == MODE_FE) {
+    double v0[5], un[5];
+    load5(a.Vin, c, v0);
+    eos_p2c(E, v0, un);
+    if (MODE == MODE_STAGE1) store5(a.Un, c, un);
+#pragma unroll
+    for (int p = 0; p < 5; p++) u[p] = un[p] + dt * r[p];
+  } else {
+    double u1[5], un[5];
+#pragma unroll
+    for (int p = 0; p < 5; p++) { u1[p] = a.U1(p, c); un[p] = a.Un(p, c); }
+    if (MODE == MODE_RK2_FINAL) {
+      const double h = 0.5 * dt;
+#pragma unroll
+      for (int p = 0; p < 5; p++) { u[p] = 0.5 * u1[p] + 0.5 * un[p]; u[p] = u[p] + h * r[p]; }
+    } else if (MODE == MODE_RK3_STAGE2) {
+      const double h = 0.25 * dt;
+#pragma unroll
+      for (int p = 0; p < 5; p++) { u[p] = 0.25 * u1[p] + 0.75 * un[p]; u[p] = u[p] + h * r[p]; }
+    } else {
+      const double h = 2.0 / 3.0 * dt;
+#pragma unroll
+      for (int p = 0; p < 5; p++) { u[p] = 2.0 / 3.0 * u1[p] + 1.0 / 3.0 * un[p]; u[p] = u[p] + h * r[p]; }
+    }
+  }
+  eos_c2p(E, u, v);
+  const bool clipped = eos_clip(E, v);
+  if (clipped) {
+    atomicAdd(&a.cnt->clipped, 1ull);
+    if (MODE == MODE_STAGE1 || MODE == MODE_RK3_STAGE2) atomicAdd(&a.cnt->stage_clipped, 1ull);
+  }
+  if (eos_check5(E, v)) atomicOr(&a.cnt->error, 1);
+  if (MODE == MODE_STAGE1 || MODE == MODE_RK3_STAGE2) store5(a.U1, c, u);
+  store5(a.Vout, c, v);
+  write_ghosts(a.g, a.Vout, i, j, k, v);
+}
 
 // One tile of the fused stage (the body of k_stage and k_stage_multi).
 // GEN: reconstruction in any variable type (false: primitive variables only,
@@ -266,48 +317,7 @@ __device__ __forceinline__ void stage_tile(const StageArgs& a, int tile) {
     r[p] = acc * cst;
   }
 
-  if (MODE == MODE_RESIDUAL) {
-    store5(a.R, c, r);
-    return;
-  }
-  const DevEos& E = M.m[myid];
-  const double dt = a.cnt->dt;
-  double u[5], v[5];
-  if (MODE == MODE_STAGE1 || MODE == MODE_FE) {
-    double v0[5], un[5];
-    load5(a.Vin, c, v0);
-    eos_p2c(E, v0, un);
-    if (MODE == MODE_STAGE1) store5(a.Un, c, un);
-#pragma unroll
-    for (int p = 0; p < 5; p++) u[p] = un[p] + dt * r[p];
-  } else {
-    double u1[5], un[5];
-#pragma unroll
-    for (int p = 0; p < 5; p++) { u1[p] = a.U1(p, c); un[p] = a.Un(p, c); }
-    if (MODE == MODE_RK2_FINAL) {
-      const double h = 0.5 * dt;
-#pragma unroll
-      for (int p = 0; p < 5; p++) { u[p] = 0.5 * u1[p] + 0.5 * un[p]; u[p] = u[p] + h * r[p]; }
-    } else if (MODE == MODE_RK3_STAGE2) {
-      const double h = 0.25 * dt;
-#pragma unroll
-      for (int p = 0; p < 5; p++) { u[p] = 0.25 * u1[p] + 0.75 * un[p]; u[p] = u[p] + h * r[p]; }
-    } else {
-      const double h = 2.0 / 3.0 * dt;
-#pragma unroll
-      for (int p = 0; p < 5; p++) { u[p] = 2.0 / 3.0 * u1[p] + 1.0 / 3.0 * un[p]; u[p] = u[p] + h * r[p]; }
-    }
-  }
-  eos_c2p(E, u, v);
-  const bool clipped = eos_clip(E, v);
-  if (clipped) {
-    atomicAdd(&a.cnt->clipped, 1ull);
-    if (MODE == MODE_STAGE1 || MODE == MODE_RK3_STAGE2) atomicAdd(&a.cnt->stage_clipped, 1ull);
-  }
-  if (eos_check5(E, v)) atomicOr(&a.cnt->error, 1);
-  if (MODE == MODE_STAGE1 || MODE == MODE_RK3_STAGE2) store5(a.U1, c, u);
-  store5(a.Vout, c, v);
-  write_ghosts(g, a.Vout, i, j, k, v);
+  stage_update<MODE>(a, M.m[myid], i, j, k, c, r);
 }
 
 // XCD-aware tile order: work-groups are dealt round-robin to the 8 XCDs,
@@ -335,6 +345,17 @@ __global__ void __launch_bounds__(BX * BY * BZ) k_stage(StageArgs a) {
   stage_tile<MODE, BX, BY, BZ, GEN>(ar, tile);
 }
 
+// member m with toff[m] <= t < toff[m+1]
+__device__ __forceinline__ int multi_member(const int* __restrict__ toff, int nm, int t) {
+  int lo = 0, hi = nm - 1;
+  while (lo < hi) {
+    const int mid = (lo + hi + 1) >> 1;
+    if (toff[mid] <= t) lo = mid;
+    else hi = mid - 1;
+  }
+  return lo;
+}
+
 // Ensemble form: the tiles of many solvers (one table entry each, the same
 // stage mode) in one launch.  toff holds the prefix sums of the members'
 // tile counts; the concatenated tile list is dealt to the XCDs as above, so
@@ -346,13 +367,8 @@ __global__ void __launch_bounds__(BX * BY * BZ) k_stage_multi(const StageArgs* _
   const int total = toff[nm];
   const int t = xcd_tile(total);
   if (t >= total) return;
-  int lo = 0, hi = nm - 1;  // member m with toff[m] <= t < toff[m+1]
-  while (lo < hi) {
-    const int mid = (lo + hi + 1) >> 1;
-    if (toff[mid] <= t) lo = mid;
-    else hi = mid - 1;
-  }
-  stage_tile<MODE, BX, BY, BZ, false>(tab[lo], t - toff[lo]);
+  const int m = multi_member(toff, nm, t);
+  stage_tile<MODE, BX, BY, BZ, false>(tab[m], t - toff[m]);
 }
 
 // Cells whose reconstruction in the scheme's variable type fails CheckState
@@ -542,9 +558,15 @@ __global__ void k_soa_to_aos(CF5 src, double* __restrict__ dst, int dof, long n)
   for (long c = blockIdx.x * (long)blockDim.x + threadIdx.x; c < n; c += (long)gridDim.x * blockDim.x)
     for (int p = 0; p < dof; p++) dst[c * dof + p] = src(p, c);
 }
-__global__ void k_i32_to_u8(const int* __restrict__ src, unsigned char* __restrict__ dst, long n) {
-  for (long c = blockIdx.x * (long)blockDim.x + threadIdx.x; c < n; c += (long)gridDim.x * blockDim.x)
+// `seen` is set once some cell holds the material `inactive`
+__global__ void k_i32_to_u8(const int* __restrict__ src, unsigned char* __restrict__ dst, long n, int inactive,
+                            int* seen) {
+  bool any = false;
+  for (long c = blockIdx.x * (long)blockDim.x + threadIdx.x; c < n; c += (long)gridDim.x * blockDim.x) {
     dst[c] = (unsigned char)src[c];
+    any |= (int)(unsigned char)src[c] == inactive;
+  }
+  if (any) *seen = 1;
 }
 __global__ void k_u8_to_i32(const unsigned char* __restrict__ src, int* __restrict__ dst, long n) {
   for (long c = blockIdx.x * (long)blockDim.x + threadIdx.x; c < n; c += (long)gridDim.x * blockDim.x)

@@ -13,6 +13,7 @@
 #pragma once
 #include <hip/hip_runtime.h>
 #include <cfloat>
+#include <cmath>
 #include "../../include/m2c_amd.h"
 
 namespace m2c {
@@ -46,6 +47,17 @@ __host__ inline DevEos make_eos(const m2cx_material& mm) {
   e.Gamma0_rho0 = mm.Gamma0 * mm.rho0;
   e.d_rho = mm.dummy_rho; e.d_p = mm.dummy_p; e.d_e = mm.dummy_e;
   return e;
+}
+
+// Parameters for which states in the range that the fast arithmetic of
+// m2c_stage_u.h checks give intermediate values in range too.
+__host__ inline bool eos_in_range(const DevEos& e) {
+  auto in = [](double x) { return std::fabs(x) >= 0x1p-100 && std::fabs(x) <= 0x1p100; };
+  auto in0 = [&](double x) { return x == 0.0 || in(x); };
+  if (e.type == M2CX_EOS_SG || e.type == M2CX_EOS_NASG)
+    return in(e.gam) && in(e.gam1) && in0(e.pc) && (e.type == M2CX_EOS_SG || (in0(e.b) && in0(e.q)));
+  if (e.type == M2CX_EOS_MG) return in(e.rho0) && in(e.c0) && in(e.Gamma0) && in0(e.s) && in0(e.e0);
+  return true;
 }
 
 // ---------------------------------------------------------------- EOS

@@ -1,0 +1,163 @@
+"""The stage on tiles of one material and on mixed tiles, against the oracle,
+bit for bit: every flux, limiter, equation of state and boundary condition on
+grids that tiles do not divide, thinner than a tile and its halo, with
+inactive cells in a one-material solver, with states at the ends of the fast
+arithmetic's range, and shock-bubbles whose grids hold both kinds of tile."""
+import numpy as np
+import pytest
+
+import oracle_lib as ol
+from m2c_amd import abi, configs
+
+pytestmark = pytest.mark.gpu
+
+MATS = {
+    "sg": abi.material("SG", gamma=1.4),
+    "stiff": abi.material("SG", gamma=6.12, pc=3.43, pmin=-3.0),
+    "nasg": abi.material("NASG", gamma=1.19, pc=6.2, b=0.05, q=-1.2),
+    "mg": abi.material("MG", rho0=1.0, c0=2.0, s=1.3, Gamma0=1.2),
+}
+BCS = (abi.BC_INLET, abi.BC_OUTLET, abi.BC_SYMMETRY, abi.BC_SLIPWALL, abi.BC_STICKWALL, abi.BC_INLET2)
+
+
+def _inner(a):
+    return a[1:-1, 1:-1, 1:-1]
+
+
+def _state(n, seed, rough):
+    rng = np.random.default_rng(seed)
+    V = np.zeros((n[2] + 2, n[1] + 2, n[0] + 2, 5))
+    amp = 0.3 if rough else 0.02
+    V[..., 0] = 1.1 * np.exp(rng.uniform(-amp, amp, V.shape[:3]))
+    V[..., 1:4] = rng.uniform(-amp, amp, V.shape[:3] + (3,)) + (2.5 if rough else 0.0) * np.array([1.0, -1.0, 0.5])
+    V[..., 4] = np.exp(rng.uniform(-amp, amp, V.shape[:3]))
+    return V
+
+
+def _pair(n, mat, V, ID=None, nmat=1, **kw):
+    from m2c_amd import runtime
+    g = abi.grid(n, (0, 0, 0), tuple(0.1 * a for a in n), BCS, inlet=[1.0, 0.2, 0.1, -0.1, 1.2],
+                 inlet2=[1.2, -0.1, 0.3, 0.2, 0.9])
+    mats = abi.materials(mat)
+    s = abi.default_scheme(**kw)
+    if ID is None:
+        ID = np.zeros(V.shape[:3], dtype=np.int32)
+    configs.fill_ghosts(V, ID, None, g)
+    o = ol.Oracle(g, mats, nmat, s)
+    o.set_state(V, ID, None)
+    gpu = runtime.Solver(g, mats, nmat, s)
+    gpu.set_state(V, ID, None)
+    return gpu, o
+
+
+def _same_residual(gpu, o):
+    try:
+        Ro = _inner(o.residual())
+    except RuntimeError as e:
+        from m2c_amd import runtime
+        assert "hyperbolicity" in str(e)
+        with pytest.raises(runtime.M2CError, match="error -4"):
+            gpu.compute_residual()
+        return
+    Rg = _inner(gpu.compute_residual())
+    assert np.array_equal(Rg, Ro, equal_nan=True), np.nanmax(np.abs(Rg - Ro))
+
+
+@pytest.mark.parametrize("mat", list(MATS))
+@pytest.mark.parametrize("flux", [abi.FLUX_HLLC, abi.FLUX_ROE, abi.FLUX_LLF])
+@pytest.mark.parametrize("limiter", [abi.LIM_VANALBADA, abi.LIM_GMM, abi.LIM_NONE])
+@pytest.mark.parametrize("rough", [False, True])
+def test_one_material(mat, flux, limiter, rough):
+    n = (35, 11, 9)
+    gpu, o = _pair(n, MATS[mat], _state(n, 5, rough), flux=flux, limiter=limiter)
+    for v in range(4):
+        gpu.set_tile(v)
+        _same_residual(gpu, o)
+
+
+@pytest.mark.parametrize("n", [(1, 1, 1), (2, 1, 1), (1, 3, 1), (1, 1, 5), (33, 1, 1), (8, 8, 4), (9, 9, 5), (7, 65, 3)])
+@pytest.mark.parametrize("ti", [abi.TI_FE, abi.TI_RK2, abi.TI_RK3])
+def test_small_and_ragged_grids(n, ti):
+    gpu, o = _pair(n, MATS["stiff"], _state(n, 8, False), integrator=ti, time_step=2e-3)
+    for v in range(4):
+        gpu.set_tile(v)
+        gpu.run_steps(1)
+        o.run_steps(1)
+        assert np.array_equal(_inner(gpu.get_state()[0]), _inner(o.get_state()[0])), v
+
+
+def test_inactive_cells_in_a_one_material_solver():
+    """Material number nmat marks inactive cells; a solver of one material
+    learns of them when the IDs are uploaded, also between steps."""
+    n = (40, 18, 13)
+    V = _state(n, 3, False)
+    gpu, o = _pair(n, MATS["sg"], V, integrator=abi.TI_RK2, cfl=0.3)
+    gpu.run_steps(1)
+    o.run_steps(1)
+    assert np.array_equal(_inner(gpu.get_state()[0]), _inner(o.get_state()[0]))
+    ID = np.zeros(V.shape[:3], dtype=np.int32)
+    ID[5:8, 7:9, 20:23] = 1
+    ID[:, 3, 3] = 1
+    gpu.upload(abi.FIELD_ID, ID)
+    o.set_state(o.get_state()[0], ID, None)
+    live = _inner(ID) == 0
+    for v in range(4):
+        gpu.set_tile(v)
+        _g, _o = _inner(gpu.compute_residual()), _inner(o.residual())
+        assert np.array_equal(_g[live], _o[live]), v
+
+
+@pytest.mark.parametrize("case", ["denormal", "tiny", "huge", "vacuum", "zeros"])
+def test_ends_of_the_fast_range(case):
+    """Velocities down to denormals (a wave's exponential front), states far
+    outside the range that the fast arithmetic takes, and exact zeros."""
+    n = (24, 10, 8)
+    rng = np.random.default_rng(2)
+    V = _state(n, 4, False)
+    mag = rng.uniform(-1, 1, V.shape[:3] + (3,))
+    if case == "denormal":
+        V[..., 1:4] = mag * 10.0 ** rng.uniform(-323, -280, mag.shape)
+    elif case == "tiny":
+        V[..., 1:4] = mag * 10.0 ** rng.uniform(-300, -100, mag.shape)
+        V[..., 4] *= 10.0 ** rng.uniform(-200, 0, V.shape[:3])
+    elif case == "huge":
+        V[..., 0] *= 1e60
+        V[..., 4] *= 1e90
+        V[..., 1:4] *= 1e15
+    elif case == "vacuum":
+        thin = 10.0 ** rng.uniform(-40, 0, V.shape[:3])
+        V[..., 0] *= thin
+        V[..., 4] *= thin
+    else:
+        V[..., 1:4] = 0.0
+        V[:, :, 12:, 0], V[:, :, :12, 0] = 1.0, 0.5
+        V[..., 4] = 1.0
+    gpu, o = _pair(n, MATS["sg"], V)
+    _same_residual(gpu, o)
+
+
+@pytest.mark.parametrize("water", ["sg", "nasg"])
+@pytest.mark.parametrize("variant", [0, 1, 2, 3])
+def test_mixed_and_one_material_tiles(water, variant):
+    """40^3 shock-bubble: tiles inside the gas, tiles of water and mixed ones,
+    with the stage overlapped with the Riemann solve and after it."""
+    from m2c_amd import runtime
+    g, mats, nmat, s, V, ID, Phi = configs.c2_shock_bubble(40, radius=0.27)
+    if water == "nasg":
+        mats[0] = abi.material("NASG", **configs.WATER_NASG)
+        r2, u2, p2 = configs.nasg_post_shock(1000.0, 1e5, *(configs.WATER_NASG[k] for k in ("gamma", "pc", "b", "q")),
+                                             1.5)
+        V[V[..., 1] > 0] = [r2, u2, 0.0, 0.0, p2]
+    o = ol.Oracle(g, mats, nmat, s)
+    o.set_state(V, ID, Phi)
+    o.run_steps(3)
+    Vo, IDo, Po = o.get_state()
+    for overlap in (True, False):
+        gpu = runtime.Solver(g, mats, nmat, s)
+        gpu.set_overlap(overlap)
+        gpu.set_tile(variant)
+        gpu.set_state(V, ID, Phi)
+        gpu.run_steps(3)
+        Vg, IDg, Pg = gpu.get_state()
+        assert np.array_equal(_inner(IDg), _inner(IDo)) and np.array_equal(_inner(Pg), _inner(Po))
+        assert np.array_equal(_inner(Vg), _inner(Vo)), np.abs(_inner(Vg) - _inner(Vo)).max()
