@@ -6,11 +6,19 @@
 set -e
 cd "$(dirname "$0")"
 HIPCC=${HIPCC:-/opt/rocm/bin/hipcc}
-$HIPCC --offload-arch=gfx950 -O3 -std=c++17 -fPIC -shared \
-  -ffp-contract=off -fno-fast-math \
-  -Xclang -target-feature -Xclang -packed-fp32-ops \
-  -Wall -Wno-unused-variable -Wno-unused-but-set-variable -Wno-unused-value -Wno-unused-result \
-  -I../include -o libm2c_amd.so.tmp csrc/m2c_capi.hip "$@"
+FLAGS="--offload-arch=gfx950 -O3 -std=c++17 -fPIC -ffp-contract=off -fno-fast-math
+  -Xclang -target-feature -Xclang -packed-fp32-ops
+  -Wall -Wno-unused-variable -Wno-unused-but-set-variable -Wno-unused-value -Wno-unused-result
+  -Wno-bitwise-instead-of-logical -I../include"
+mkdir -p build
+pids=()
+UNITS="m2c_capi m2c_stage m2c_stage_u m2c_stage_ur"
+for unit in $UNITS; do
+  $HIPCC $FLAGS -c -o build/$unit.o csrc/$unit.hip "$@" &
+  pids+=($!)
+done
+for p in "${pids[@]}"; do wait "$p"; done
+$HIPCC --offload-arch=gfx950 -fPIC -shared -o libm2c_amd.so.tmp $(printf 'build/%s.o ' $UNITS)
 # replace the library in one step, so that a reader never sees a partial file
 mv -f libm2c_amd.so.tmp libm2c_amd.so
 # C++ facades with the reference's SpaceVariable3D / SpaceOperator /

@@ -13,7 +13,8 @@
 #include <tuple>
 #include <string>
 #include <vector>
-#include "m2c_stage_u.h"
+#include "m2c_stage_launch.h"
+#include "m2c_kernels.h"
 #include "m2c_multiphase.h"
 #include "m2c_reinit.h"
 #include "m2c_band.h"
@@ -28,12 +29,6 @@ struct Timer {
   double ms = 0.0;
   long long launches = 0;
 };
-
-// Stage-kernel tile shapes the autotuner chooses from (all 256 threads).
-struct TileVariant {
-  int bx, by, bz;
-};
-static const TileVariant kTiles[] = {{16, 4, 4}, {32, 4, 2}, {8, 8, 4}, {16, 8, 2}};
 
 // A level set after the first (m2cx_create_levelsets): the fields, settings
 // and reinitializer state the solver's own members hold for level set 0,
@@ -244,6 +239,9 @@ static int mat_slot_acquire(m2cx_solver* h) {
   if (slot < 0) return fail(h, M2CX_E_CAPACITY, "too many distinct material tables on one device");
   if (v[slot].refs == 0) {
     hipError_t e = hipMemcpyToSymbol(HIP_SYMBOL(c_mats), &h->M, sizeof(DevMats), slot * sizeof(DevMats));
+    if (e == hipSuccess) e = stage_set_materials(slot, h->M);
+    if (e == hipSuccess) e = ustage_set_materials_hllc(slot, h->M);
+    if (e == hipSuccess) e = ustage_set_materials_other(slot, h->M);
     if (e != hipSuccess) return fail(h, M2CX_E_HIP, std::string("material table upload: ") + hipGetErrorString(e));
     v[slot].m = h->M;
   }
@@ -633,7 +631,7 @@ static int create_impl(const m2cx_grid* grid, const m2cx_material* mats, int nma
   }
   long mt = 0;
   for (const TileVariant& t : kTiles)
-    mt = std::max(mt, (long)((NX + t.bx - 1) / t.bx) * ((NY + t.by - 1) / t.by) * ((NZ + t.bz - 1) / t.bz));
+    mt = std::max(mt, stage_tiles(g, t.bx, t.by, t.bz));
   HIPCHK(h, hipMalloc(&h->tflag, mt));
   // the one-material stage kernel: what its code leaves out (m2c_stage_u.h)
   h->ustage = s.flux != M2CX_FLUX_GODUNOV && s.rec_type == M2CX_REC_LINEAR && s.var_type == M2CX_VAR_PRIMITIVE;
@@ -821,67 +819,12 @@ static StageArgs stage_args(m2cx_solver* h, int vin, int vout, int mode) {
 }
 
 extern "C++" {
-static constexpr int kNumTiles = 4;
-
-// one work-group per tile, padded to a multiple of the XCD count (see
-// xcd_tile for the tile order)
-template <int BX, int BY, int BZ>
-static dim3 stage_grid(const DevGrid& g) {
-  const long ntiles = (long)((g.NX + BX - 1) / BX) * ((g.NY + BY - 1) / BY) * ((g.NZ + BZ - 1) / BZ);
-  return dim3((unsigned)((ntiles + NXCD - 1) / NXCD * NXCD));
-}
-
-template <int BX, int BY, int BZ, bool GEN>
-static void launch_stage_tile(m2cx_solver* h, const StageArgs& a, int mode, hipStream_t st) {
-  const dim3 grid = stage_grid<BX, BY, BZ>(h->g);
-  constexpr int nt = BX * BY * BZ;
-  switch (mode) {
-    case MODE_RESIDUAL: k_stage<MODE_RESIDUAL, BX, BY, BZ, GEN><<<grid, nt, 0, st>>>(a); break;
-    case MODE_STAGE1: k_stage<MODE_STAGE1, BX, BY, BZ, GEN><<<grid, nt, 0, st>>>(a); break;
-    case MODE_RK2_FINAL: k_stage<MODE_RK2_FINAL, BX, BY, BZ, GEN><<<grid, nt, 0, st>>>(a); break;
-    case MODE_RK3_STAGE2: k_stage<MODE_RK3_STAGE2, BX, BY, BZ, GEN><<<grid, nt, 0, st>>>(a); break;
-    case MODE_RK3_FINAL: k_stage<MODE_RK3_FINAL, BX, BY, BZ, GEN><<<grid, nt, 0, st>>>(a); break;
-    case MODE_FE: k_stage<MODE_FE, BX, BY, BZ, GEN><<<grid, nt, 0, st>>>(a); break;
-  }
-}
-
-template <int BX, int BY, int BZ>
-static void launch_ustage_tile(m2cx_solver* h, const StageArgs& a, int mode, hipStream_t st) {
-  const dim3 grid = stage_grid<BX, BY, BZ>(h->g);
-  constexpr int nt = BX * BY * BZ;
-  switch (mode) {
-    case MODE_RESIDUAL: k_stage_u<MODE_RESIDUAL, BX, BY, BZ><<<grid, nt, 0, st>>>(a); break;
-    case MODE_STAGE1: k_stage_u<MODE_STAGE1, BX, BY, BZ><<<grid, nt, 0, st>>>(a); break;
-    case MODE_RK2_FINAL: k_stage_u<MODE_RK2_FINAL, BX, BY, BZ><<<grid, nt, 0, st>>>(a); break;
-    case MODE_RK3_STAGE2: k_stage_u<MODE_RK3_STAGE2, BX, BY, BZ><<<grid, nt, 0, st>>>(a); break;
-    case MODE_RK3_FINAL: k_stage_u<MODE_RK3_FINAL, BX, BY, BZ><<<grid, nt, 0, st>>>(a); break;
-    case MODE_FE: k_stage_u<MODE_FE, BX, BY, BZ><<<grid, nt, 0, st>>>(a); break;
-  }
-}
-
-static void launch_ustage_variant(m2cx_solver* h, const StageArgs& a, int mode, int v, hipStream_t st) {
-  switch (v) {
-    case 1: launch_ustage_tile<32, 4, 2>(h, a, mode, st); break;
-    case 2: launch_ustage_tile<8, 8, 4>(h, a, mode, st); break;
-    case 3: launch_ustage_tile<16, 8, 2>(h, a, mode, st); break;
-    default: launch_ustage_tile<16, 4, 4>(h, a, mode, st); break;
-  }
-}
-
 // Reconstruction in conservative or characteristic variables runs one tile
 // shape (16x4x4) of the general kernel; primitive variables choose the tuned
 // tile of the primitive-only kernel.
 static void launch_stage_variant(m2cx_solver* h, const StageArgs& a, int mode, int v, hipStream_t st) {
-  if (a.s.var_type != M2CX_VAR_PRIMITIVE && a.s.rec_type == M2CX_REC_LINEAR) {
-    launch_stage_tile<16, 4, 4, true>(h, a, mode, st);
-    return;
-  }
-  switch (v) {
-    case 1: launch_stage_tile<32, 4, 2, false>(h, a, mode, st); break;
-    case 2: launch_stage_tile<8, 8, 4, false>(h, a, mode, st); break;
-    case 3: launch_stage_tile<16, 8, 2, false>(h, a, mode, st); break;
-    default: launch_stage_tile<16, 4, 4, false>(h, a, mode, st); break;
-  }
+  if (a.s.var_type != M2CX_VAR_PRIMITIVE && a.s.rec_type == M2CX_REC_LINEAR) stage_launch_gen(a, mode, st);
+  else stage_launch(a, mode, v, st);
 }
 
 // the tile shape the stage kernel runs with
@@ -904,7 +847,8 @@ static void launch_stage(m2cx_solver* h, int vin, int vout, int mode, int phase 
   const int v = h->tile < 0 ? 0 : h->tile;
   hipEvent_t e0{};
   tic(h, name, &e0, st);
-  if (h->ustage && phase != 2) launch_ustage_variant(h, a, mode, v, st);
+  if (h->ustage && phase != 2)
+    (a.s.flux == M2CX_FLUX_HLLC ? ustage_launch_hllc : ustage_launch_other)(a, mode, v, st);
   a.phase = (h->ustage && phase == 0) ? 2 : phase;
   if (!h->ustage || phase == 2 || (phase == 0 && a.tflag)) launch_stage_variant(h, a, mode, v, st);
   toc(h, name, e0, st);
@@ -2121,6 +2065,7 @@ struct m2cx_ensemble {
   struct StageClass {
     int v = 0;                 // tile variant (kTiles index)
     bool ustage = false;       // one-material tiles run k_stage_u_multi
+    bool hllc = false;         // compiled for the HLLC flux
     std::vector<m2cx_solver*> members;
     StageArgs* tab[3][2] = {};
     int* toff = nullptr;
@@ -2149,56 +2094,14 @@ static bool ens_riemann_member(const m2cx_solver* h) {
   return h->multimat && h->sch.mp_flux != M2CX_MPFLUX_LLF;
 }
 
-extern "C++" {
-// k_stage_multi (k_stage_u_multi) for one class, stage and phase (1: tiles of
-// one material, 2: the mixed ones) on stream `st`
-template <int BX, int BY, int BZ>
-static void launch_class_tile(const m2cx_ensemble::StageClass& c, const StageArgs* tab, int mode, hipStream_t st) {
-  const long per = ((long)c.ntiles + NXCD - 1) / NXCD;
-  const dim3 grid((unsigned)(per * NXCD));
-  const int nm = (int)c.members.size();
-  constexpr int nt = BX * BY * BZ;
-  switch (mode) {
-    case MODE_STAGE1: k_stage_multi<MODE_STAGE1, BX, BY, BZ><<<grid, nt, 0, st>>>(tab, c.toff, nm); break;
-    case MODE_RK2_FINAL: k_stage_multi<MODE_RK2_FINAL, BX, BY, BZ><<<grid, nt, 0, st>>>(tab, c.toff, nm); break;
-    case MODE_RK3_STAGE2: k_stage_multi<MODE_RK3_STAGE2, BX, BY, BZ><<<grid, nt, 0, st>>>(tab, c.toff, nm); break;
-    case MODE_RK3_FINAL: k_stage_multi<MODE_RK3_FINAL, BX, BY, BZ><<<grid, nt, 0, st>>>(tab, c.toff, nm); break;
-  }
-}
-template <int BX, int BY, int BZ>
-static void launch_class_utile(const m2cx_ensemble::StageClass& c, const StageArgs* tab, int mode, hipStream_t st) {
-  const long per = ((long)c.ntiles + NXCD - 1) / NXCD;
-  const dim3 grid((unsigned)(per * NXCD));
-  const int nm = (int)c.members.size();
-  constexpr int nt = BX * BY * BZ;
-  switch (mode) {
-    case MODE_STAGE1: k_stage_u_multi<MODE_STAGE1, BX, BY, BZ><<<grid, nt, 0, st>>>(tab, c.toff, nm); break;
-    case MODE_RK2_FINAL: k_stage_u_multi<MODE_RK2_FINAL, BX, BY, BZ><<<grid, nt, 0, st>>>(tab, c.toff, nm); break;
-    case MODE_RK3_STAGE2: k_stage_u_multi<MODE_RK3_STAGE2, BX, BY, BZ><<<grid, nt, 0, st>>>(tab, c.toff, nm); break;
-    case MODE_RK3_FINAL: k_stage_u_multi<MODE_RK3_FINAL, BX, BY, BZ><<<grid, nt, 0, st>>>(tab, c.toff, nm); break;
-  }
-}
-
+// the stage of one class's members in one launch (phase 1: tiles of one
+// material, 2: the mixed ones)
 static void launch_class(const m2cx_ensemble::StageClass& c, int q, int phase, int mode, hipStream_t st) {
-  const StageArgs* tab = c.tab[q][phase - 1];
-  if (c.ustage && phase == 1) {
-    switch (c.v) {
-      case 1: launch_class_utile<32, 4, 2>(c, tab, mode, st); break;
-      case 2: launch_class_utile<8, 8, 4>(c, tab, mode, st); break;
-      case 3: launch_class_utile<16, 8, 2>(c, tab, mode, st); break;
-      default: launch_class_utile<16, 4, 4>(c, tab, mode, st); break;
-    }
-    return;
-  }
-  switch (c.v) {
-    case 1: launch_class_tile<32, 4, 2>(c, tab, mode, st); break;
-    case 2: launch_class_tile<8, 8, 4>(c, tab, mode, st); break;
-    case 3: launch_class_tile<16, 8, 2>(c, tab, mode, st); break;
-    default: launch_class_tile<16, 4, 4>(c, tab, mode, st); break;
-  }
+  const int nm = (int)c.members.size();
+  if (c.ustage && phase == 1)
+    (c.hllc ? ustage_launch_multi_hllc : ustage_launch_multi_other)(c.tab[q][0], c.toff, nm, c.ntiles, mode, c.v, st);
+  else stage_launch_multi(c.tab[q][phase - 1], c.toff, nm, c.ntiles, mode, c.v, st);
 }
-
-}  // extern "C++"
 
 static void free_classes(m2cx_ensemble* e) {
   for (auto& c : e->classes) {
@@ -2321,15 +2224,17 @@ static int ensemble_build(m2cx_ensemble* e) {
   free_classes(e);
   e->classed.clear();
   if (e->overlap) {
-    std::map<std::pair<int, bool>, m2cx_ensemble::StageClass> bytile;
+    std::map<std::tuple<int, bool, bool>, m2cx_ensemble::StageClass> bytile;
     for (size_t i = 0; i < e->m.size(); i++) {
       m2cx_solver* h = e->m[i];
       if (!e->active[i] || !ens_riemann_member(h)) continue;
       if (h->s.var_type != M2CX_VAR_PRIMITIVE && h->s.rec_type == M2CX_REC_LINEAR) continue;
       const int v = h->tile < 0 ? 0 : h->tile;
-      auto& c = bytile[{v, h->ustage}];
+      const bool hllc = h->s.flux == M2CX_FLUX_HLLC;
+      auto& c = bytile[{v, h->ustage, hllc}];
       c.v = v;
       c.ustage = h->ustage;
+      c.hllc = hllc;
       c.members.push_back(h);
     }
     for (auto& kv : bytile) {

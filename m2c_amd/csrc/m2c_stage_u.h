@@ -1,11 +1,11 @@
 // The fused stage on tiles of one material (gfx950): the same stage as
-// stage_tile of m2c_kernels.h, bit for bit, for tiles whose cells and the two
+// stage_tile of m2c_stage.h, bit for bit, for tiles whose cells and the two
 // cells around them along each axis all hold one active material
 // (k_tile_mixed), with a primitive (or constant) reconstruction on a uniform
 // mesh and an HLLC, Roe or LLF flux.  That is nearly every tile of a run.
 #pragma once
 #include "m2c_exactdiv.h"
-#include "m2c_kernels.h"
+#include "m2c_stage.h"
 
 namespace m2c {
 
@@ -214,10 +214,14 @@ __device__ __forceinline__ void flux_hllc_axis(const DevEos& E, bool z, const do
   err |= e1;
 }
 
-// Roe and LLF keep the x, y, z order (their sums run over it)
+// Roe and LLF keep the x, y, z order (their sums run over it).  HLLC: compiled
+// for that flux alone; the Roe flux's eigenvectors take 203 registers, two
+// waves per SIMD instead of three (256^3 water: 2.42 ms per launch against
+// 1.86 ms).
+template <bool HLLC>
 __device__ __forceinline__ void flux_axis(const DevEos& E, const Scheme& s, int D, const double* Wm, const double* Wp,
                                           double* F, int& err) {
-  if (s.flux == M2CX_FLUX_HLLC) {
+  if (HLLC) {
     flux_hllc_axis(E, D == 2, Wm, Wp, F, err);
     return;
   }
@@ -267,8 +271,10 @@ __device__ __forceinline__ void ghost_axis(int bc, const CF5& V, long cg, int D,
 //
 // Bound by FP64 issue and the latency of its chains, not by memory (200 B per
 // cell and launch are 0.7 ms of a 256^3 launch).  256^3 water, RK3 launches:
-// 4.24 ms with stage_tile, 2.42 ms here; 128x32x32 gas: 53 -> 24.5 us.
-template <int MODE, int BX, int BY, int BZ>
+// 4.24 ms with stage_tile, 1.86 ms here (VALU issue on 64% of the cycles at
+// three waves per SIMD; held to 128 registers for four it spills: 2.88 ms);
+// 128x32x32 gas: 53 -> 24 us.
+template <int MODE, int BX, int BY, int BZ, bool HLLC>
 __device__ __forceinline__ void ustage_body(const StageArgs& a, int tile, const DevEos E,
                                             double (*sF)[TileShape<BX, BY, BZ>::NFACE]) {
   using TS = TileShape<BX, BY, BZ>;
@@ -395,10 +401,14 @@ __device__ __forceinline__ void ustage_body(const StageArgs& a, int tile, const 
       if (pos == 0) ghost_axis(g.bc[2 * D], a.Vin, cf - axis_stride(g, D), D, Wp, Wm);
       else ghost_axis(g.bc[2 * D + 1], a.Vin, cf, D, Wm, Wp);
     }
-    flux_axis(E, s, D, Wm, Wp, F, err);
+    flux_axis<HLLC>(E, s, D, Wm, Wp, F, err);
 #pragma unroll
     for (int q = 0; q < 5; q++) sF[axis_comp(D, q)][slot] = F[q];
   }
+  // the conserved states that the combination reads, on their way while the
+  // other waves finish their fluxes
+  StageIn in;
+  if (inside) stage_load<MODE>(a, c, in);
   __syncthreads();
   if (err) atomicOr(&a.cnt->error, 1);
   if (!inside) return;
@@ -420,10 +430,10 @@ __device__ __forceinline__ void ustage_body(const StageArgs& a, int tile, const 
     acc = acc + az * sF[p][fzp];
     r[p] = acc * cst;
   }
-  stage_update<MODE>(a, E, i, j, k, c, r);
+  stage_update<MODE>(a, E, in, i, j, k, c, r);
 }
 
-template <int MODE, int BX, int BY, int BZ>
+template <int MODE, int BX, int BY, int BZ, bool HLLC>
 __device__ __forceinline__ void ustage_tile(const StageArgs& a, int tile) {
   __shared__ double sF[5][TileShape<BX, BY, BZ>::NFACE];
   if (a.tflag && a.tflag[tile]) return;
@@ -434,12 +444,12 @@ __device__ __forceinline__ void ustage_tile(const StageArgs& a, int tile) {
   const DevEos E = c_mats[a.s.mset].m[id];
   // one copy of the tile's code per type of equation of state, each without
   // the others' branches
-  if (E.type == M2CX_EOS_SG) ustage_body<MODE, BX, BY, BZ>(a, tile, E, sF);
-  else if (E.type == M2CX_EOS_NASG) ustage_body<MODE, BX, BY, BZ>(a, tile, E, sF);
-  else ustage_body<MODE, BX, BY, BZ>(a, tile, E, sF);
+  if (E.type == M2CX_EOS_SG) ustage_body<MODE, BX, BY, BZ, HLLC>(a, tile, E, sF);
+  else if (E.type == M2CX_EOS_NASG) ustage_body<MODE, BX, BY, BZ, HLLC>(a, tile, E, sF);
+  else ustage_body<MODE, BX, BY, BZ, HLLC>(a, tile, E, sF);
 }
 
-template <int MODE, int BX, int BY, int BZ>
+template <int MODE, int BX, int BY, int BZ, bool HLLC>
 __global__ void __launch_bounds__(BX * BY * BZ) k_stage_u(StageArgs a) {
   // read in place, as in k_stage
   const StageArgs& ar = *(const StageArgs*)__builtin_amdgcn_kernarg_segment_ptr();
@@ -447,48 +457,18 @@ __global__ void __launch_bounds__(BX * BY * BZ) k_stage_u(StageArgs a) {
   const int ntiles = ((g.NX + BX - 1) / BX) * ((g.NY + BY - 1) / BY) * ((g.NZ + BZ - 1) / BZ);
   const int tile = xcd_tile(ntiles);
   if (tile >= ntiles) return;
-  ustage_tile<MODE, BX, BY, BZ>(ar, tile);
+  ustage_tile<MODE, BX, BY, BZ, HLLC>(ar, tile);
 }
 
 // the members of an ensemble in one launch, as k_stage_multi
-template <int MODE, int BX, int BY, int BZ>
+template <int MODE, int BX, int BY, int BZ, bool HLLC>
 __global__ void __launch_bounds__(BX * BY * BZ) k_stage_u_multi(const StageArgs* __restrict__ tab,
                                                                  const int* __restrict__ toff, int nm) {
   const int total = toff[nm];
   const int t = xcd_tile(total);
   if (t >= total) return;
   const int m = multi_member(toff, nm, t);
-  ustage_tile<MODE, BX, BY, BZ>(tab[m], t - toff[m]);
-}
-
-// tflag[tile] = 1 where the tile's cells and the two cells around them along
-// each axis (the reach of the stage's stencil) do not all hold one active
-// material.  One wave per tile; the IDs change once per time step at most, so
-// this runs once per step.
-__global__ void __launch_bounds__(256) k_tile_mixed(DevGrid g, int inactive, const unsigned char* __restrict__ ID,
-                                                    unsigned char* __restrict__ tflag, int BX, int BY, int BZ,
-                                                    int ntiles) {
-  const int tile = (int)(blockIdx.x * 4 + threadIdx.x / 64), lane = threadIdx.x % 64;
-  if (tile >= ntiles) return;
-  const int ntx = (g.NX + BX - 1) / BX, nty = (g.NY + BY - 1) / BY;
-  const int ib = (tile % ntx) * BX, jb = ((tile / ntx) % nty) * BY, kb = (tile / (ntx * nty)) * BZ;
-  const int id0 = ID[gidx(g, ib, jb, kb)];
-  bool mixed = id0 == inactive;
-  // box D: the tile widened by two cells along axis D, cut to the ghosted brick
-#pragma unroll 1
-  for (int D = 0; D < 3; D++) {
-    const int i0 = D == 0 ? max(ib - 2, -1) : ib, j0 = D == 1 ? max(jb - 2, -1) : jb, k0 = D == 2 ? max(kb - 2, -1) : kb;
-    const int i1 = D == 0 ? min(ib + BX + 2, g.NX + 1) : min(ib + BX, g.NX);
-    const int j1 = D == 1 ? min(jb + BY + 2, g.NY + 1) : min(jb + BY, g.NY);
-    const int k1 = D == 2 ? min(kb + BZ + 2, g.NZ + 1) : min(kb + BZ, g.NZ);
-    const int nx = i1 - i0, nxy = nx * (j1 - j0), n = nxy * (k1 - k0);
-    for (int q = lane; q < n; q += 64) {
-      const int kk = q / nxy, r = q - kk * nxy, jj = r / nx, ii = r - jj * nx;
-      mixed = mixed || ID[gidx(g, i0 + ii, j0 + jj, k0 + kk)] != id0;
-    }
-  }
-  const bool any = __any(mixed);
-  if (lane == 0) tflag[tile] = any ? 1 : 0;
+  ustage_tile<MODE, BX, BY, BZ, HLLC>(tab[m], t - toff[m]);
 }
 
 }  // namespace m2c

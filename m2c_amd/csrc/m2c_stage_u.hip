@@ -1,0 +1,18 @@
+// The stage kernel of tiles of one material, HLLC flux.
+#include <hip/hip_runtime.h>
+#include "m2c_stage_u_launch.h"
+
+namespace m2c {
+
+void ustage_launch_hllc(const StageArgs& a, int mode, int variant, hipStream_t st) {
+  launch_shape<true>(a, mode, variant, st);
+}
+void ustage_launch_multi_hllc(const StageArgs* tab, const int* toff, int nm, int ntiles, int mode, int variant,
+                              hipStream_t st) {
+  launch_shape_multi<true>(tab, toff, nm, ntiles, mode, variant, st);
+}
+hipError_t ustage_set_materials_hllc(int slot, const DevMats& m) {
+  return hipMemcpyToSymbol(HIP_SYMBOL(c_mats), &m, sizeof(DevMats), slot * sizeof(DevMats));
+}
+
+}  // namespace m2c
