@@ -22,7 +22,7 @@ namespace m2c {
 
 struct DevEos {
   int type;
-  int pad;
+  int fast;  // SG or NASG with parameters in range (eos_in_range)
   double gam, pc, gam1, invgam1, gam_pc, b, q;
   double rho0, c0, Gamma0, s, e0, rho0_c0_c0, Gamma0_over_2, Gamma0_rho0;
   double rhomin, pmin, rhomax, pmax, failsafe;
@@ -33,6 +33,17 @@ struct DevMats {
   DevEos m[M2C_MAX_MAT + 1];  // index nmat is the inactive (dummy) material
   int nmat;
 };
+
+// Parameters for which states in the range that the fast arithmetic of
+// m2c_stage_u.h and m2c_riemann.h checks give intermediate values in range too.
+__host__ inline bool eos_in_range(const DevEos& e) {
+  auto in = [](double x) { return std::fabs(x) >= 0x1p-100 && std::fabs(x) <= 0x1p100; };
+  auto in0 = [&](double x) { return x == 0.0 || in(x); };
+  if (e.type == M2CX_EOS_SG || e.type == M2CX_EOS_NASG)
+    return in(e.gam) && in(e.gam1) && in0(e.pc) && (e.type == M2CX_EOS_SG || (in0(e.b) && in0(e.q)));
+  if (e.type == M2CX_EOS_MG) return in(e.rho0) && in(e.c0) && in(e.Gamma0) && in0(e.s) && in0(e.e0);
+  return true;
+}
 
 __host__ inline DevEos make_eos(const m2cx_material& mm) {
   DevEos e{};
@@ -45,19 +56,9 @@ __host__ inline DevEos make_eos(const m2cx_material& mm) {
   e.rho0_c0_c0 = mm.rho0 * mm.c0 * mm.c0;
   e.Gamma0_over_2 = 0.5 * mm.Gamma0;
   e.Gamma0_rho0 = mm.Gamma0 * mm.rho0;
+  e.fast = (e.type == M2CX_EOS_SG || e.type == M2CX_EOS_NASG) && eos_in_range(e);
   e.d_rho = mm.dummy_rho; e.d_p = mm.dummy_p; e.d_e = mm.dummy_e;
   return e;
-}
-
-// Parameters for which states in the range that the fast arithmetic of
-// m2c_stage_u.h checks give intermediate values in range too.
-__host__ inline bool eos_in_range(const DevEos& e) {
-  auto in = [](double x) { return std::fabs(x) >= 0x1p-100 && std::fabs(x) <= 0x1p100; };
-  auto in0 = [&](double x) { return x == 0.0 || in(x); };
-  if (e.type == M2CX_EOS_SG || e.type == M2CX_EOS_NASG)
-    return in(e.gam) && in(e.gam1) && in0(e.pc) && (e.type == M2CX_EOS_SG || (in0(e.b) && in0(e.q)));
-  if (e.type == M2CX_EOS_MG) return in(e.rho0) && in(e.c0) && in(e.Gamma0) && in0(e.s) && in0(e.e0);
-  return true;
 }
 
 // ---------------------------------------------------------------- EOS
