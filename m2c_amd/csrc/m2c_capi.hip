@@ -19,6 +19,7 @@
 #include "m2c_reinit.h"
 #include "m2c_band.h"
 #include "m2c_mlp.h"
+#include "m2c_hostcopy.h"
 #include <algorithm>
 #include <random>
 
@@ -120,6 +121,7 @@ struct m2cx_solver {
   bool profile = false;
   std::map<std::string, Timer> timers;
   std::string err;
+  HostPipe pipe;  // large copies to and from the caller's arrays
 };
 
 static int fail(m2cx_solver* h, int code, const std::string& msg) {
@@ -691,8 +693,7 @@ int m2cx_upload_levelset(m2cx_solver* h, int ls, const double* host) {
   if (ls < 0 || ls >= h->nls) return fail(h, M2CX_E_ARG, "no such level set");
   HIPCHK(h, hipSetDevice(h->device));
   double* dst = ls == 0 ? h->mp.phi : h->lsx[ls - 1].phi;
-  HIPCHK(h, hipMemcpyAsync(dst, host, h->ncells * 8, hipMemcpyHostToDevice, h->stream));
-  HIPCHK(h, hipStreamSynchronize(h->stream));
+  HIPCHK(h, h->pipe.to_device(h->device, dst, host, h->ncells * 8, h->stream));
   return 0;
 }
 
@@ -703,8 +704,7 @@ int m2cx_download_levelset(m2cx_solver* h, int ls, int what, double* host) {
   const bool own = ls == 0;
   const double* src = what == M2CX_LS_PHI ? (own ? h->mp.phi : h->lsx[ls - 1].phi)
                                           : (own ? h->mp.rls : h->lsx[ls - 1].rls);
-  HIPCHK(h, hipMemcpyAsync(host, src, h->ncells * 8, hipMemcpyDeviceToHost, h->stream));
-  HIPCHK(h, hipStreamSynchronize(h->stream));
+  HIPCHK(h, h->pipe.to_host(h->device, host, src, h->ncells * 8, h->stream));
   return 0;
 }
 
@@ -713,7 +713,7 @@ int m2cx_upload(m2cx_solver* h, int field, const void* host) {
   HIPCHK(h, hipSetDevice(h->device));
   const long n = h->ncells;
   if (field == M2CX_FIELD_ID) {
-    HIPCHK(h, hipMemcpyAsync(h->staging_i, host, n * 4, hipMemcpyHostToDevice, h->stream));
+    HIPCHK(h, h->pipe.to_device(h->device, h->staging_i, host, n * 4, h->stream));
     k_i32_to_u8<<<grid_blocks(n), 256, 0, h->stream>>>(h->staging_i, h->ID, n, h->s.inactive, &h->cnt->inactive_seen);
     if (!h->multimat) {
       int seen = 0;
@@ -723,11 +723,11 @@ int m2cx_upload(m2cx_solver* h, int field, const void* host) {
     }
   } else if (field == M2CX_FIELD_PHI) {
     if (!h->mp.phi) return fail(h, M2CX_E_ARG, "no level set");
-    HIPCHK(h, hipMemcpyAsync(h->mp.phi, host, n * 8, hipMemcpyHostToDevice, h->stream));
+    HIPCHK(h, h->pipe.to_device(h->device, h->mp.phi, host, n * 8, h->stream));
   } else {
     double** f = field_ptr(h, field);
     if (!f) return fail(h, M2CX_E_ARG, "bad field");
-    HIPCHK(h, hipMemcpyAsync(h->staging, host, n * 5 * 8, hipMemcpyHostToDevice, h->stream));
+    HIPCHK(h, h->pipe.to_device(h->device, h->staging, host, n * 5 * 8, h->stream));
     k_aos_to_soa<<<grid_blocks(n), 256, 0, h->stream>>>(h->staging, f5(h, f), 5, n);
   }
   HIPCHK(h, hipGetLastError());
@@ -741,18 +741,18 @@ int m2cx_download(m2cx_solver* h, int field, void* host) {
   const long n = h->ncells;
   if (field == M2CX_FIELD_ID) {
     k_u8_to_i32<<<grid_blocks(n), 256, 0, h->stream>>>(h->ID, h->staging_i, n);
-    HIPCHK(h, hipMemcpyAsync(host, h->staging_i, n * 4, hipMemcpyDeviceToHost, h->stream));
+    HIPCHK(h, hipGetLastError());
+    HIPCHK(h, h->pipe.to_host(h->device, host, h->staging_i, n * 4, h->stream));
   } else if (field == M2CX_FIELD_PHI) {
     if (!h->mp.phi) return fail(h, M2CX_E_ARG, "no level set");
-    HIPCHK(h, hipMemcpyAsync(host, h->mp.phi, n * 8, hipMemcpyDeviceToHost, h->stream));
+    HIPCHK(h, h->pipe.to_host(h->device, host, h->mp.phi, n * 8, h->stream));
   } else {
     double** f = field_ptr(h, field);
     if (!f) return fail(h, M2CX_E_ARG, "bad field");
     k_soa_to_aos<<<grid_blocks(n), 256, 0, h->stream>>>(cf5(h, f), h->staging, 5, n);
-    HIPCHK(h, hipMemcpyAsync(host, h->staging, n * 5 * 8, hipMemcpyDeviceToHost, h->stream));
+    HIPCHK(h, hipGetLastError());
+    HIPCHK(h, h->pipe.to_host(h->device, host, h->staging, n * 5 * 8, h->stream));
   }
-  HIPCHK(h, hipGetLastError());
-  HIPCHK(h, hipStreamSynchronize(h->stream));
   return 0;
 }
 
@@ -2026,7 +2026,8 @@ int m2cx_levelset_residual(m2cx_solver* h, int v_field) {
 
 int m2cx_download_ls_residual(m2cx_solver* h, double* host) {
   if (!h || !h->mp.rls) return M2CX_E_ARG;
-  HIPCHK(h, hipMemcpy(host, h->mp.rls, h->ncells * 8, hipMemcpyDeviceToHost));
+  HIPCHK(h, hipSetDevice(h->device));
+  HIPCHK(h, h->pipe.to_host(h->device, host, h->mp.rls, h->ncells * 8, h->stream));
   return 0;
 }
 
