@@ -12,7 +12,7 @@ FLAGS="--offload-arch=gfx950 -O3 -std=c++17 -fPIC -ffp-contract=off -fno-fast-ma
   -Wno-bitwise-instead-of-logical -I../include"
 mkdir -p build
 pids=()
-UNITS="m2c_capi m2c_stage m2c_stage_u m2c_stage_ur"
+UNITS="m2c_capi m2c_stage m2c_stage_u m2c_stage_ur m2c_stage_ug"
 for unit in $UNITS; do
   $HIPCC $FLAGS -c -o build/$unit.o csrc/$unit.hip "$@" &
   pids+=($!)

@@ -244,6 +244,7 @@ static int mat_slot_acquire(m2cx_solver* h) {
     if (e == hipSuccess) e = stage_set_materials(slot, h->M);
     if (e == hipSuccess) e = ustage_set_materials_hllc(slot, h->M);
     if (e == hipSuccess) e = ustage_set_materials_other(slot, h->M);
+    if (e == hipSuccess) e = ustage_set_materials_gen(slot, h->M);
     if (e != hipSuccess) return fail(h, M2CX_E_HIP, std::string("material table upload: ") + hipGetErrorString(e));
     v[slot].m = h->M;
   }
@@ -636,7 +637,7 @@ static int create_impl(const m2cx_grid* grid, const m2cx_material* mats, int nma
     mt = std::max(mt, stage_tiles(g, t.bx, t.by, t.bz));
   HIPCHK(h, hipMalloc(&h->tflag, mt));
   // the one-material stage kernel: what its code leaves out (m2c_stage_u.h)
-  h->ustage = s.flux != M2CX_FLUX_GODUNOV && s.rec_type == M2CX_REC_LINEAR && s.var_type == M2CX_VAR_PRIMITIVE;
+  h->ustage = s.flux != M2CX_FLUX_GODUNOV && s.rec_type == M2CX_REC_LINEAR;
   for (size_t q = 0; q < Acoef.size(); q++)
     h->ustage = h->ustage && Acoef[q] == 1.0 && Bcoef[q] == 1.0 && (s.limiter != M2CX_LIM_VANALBADA || Kcoef[q] == 2);
   for (int q = 0; q < nmat; q++) h->ustage = h->ustage && eos_in_range(M.m[q]);
@@ -820,7 +821,7 @@ static StageArgs stage_args(m2cx_solver* h, int vin, int vout, int mode) {
 
 extern "C++" {
 // Reconstruction in conservative or characteristic variables runs one tile
-// shape (16x4x4) of the general kernel; primitive variables choose the tuned
+// shape (kGenTile) of the general kernel; primitive variables choose the tuned
 // tile of the primitive-only kernel.
 static void launch_stage_variant(m2cx_solver* h, const StageArgs& a, int mode, int v, hipStream_t st) {
   if (a.s.var_type != M2CX_VAR_PRIMITIVE && a.s.rec_type == M2CX_REC_LINEAR) stage_launch_gen(a, mode, st);
@@ -830,7 +831,8 @@ static void launch_stage_variant(m2cx_solver* h, const StageArgs& a, int mode, i
 // the tile shape the stage kernel runs with
 static void stage_tile_dims(const m2cx_solver* h, int& tx, int& ty, int& tz) {
   if (h->s.var_type != M2CX_VAR_PRIMITIVE && h->s.rec_type == M2CX_REC_LINEAR) {
-    tx = 16; ty = 4; tz = 4;
+    const TileVariant& t = kTiles[kGenTile];
+    tx = t.bx; ty = t.by; tz = t.bz;
     return;
   }
   const TileVariant& t = kTiles[h->tile < 0 ? 0 : h->tile];
@@ -847,8 +849,10 @@ static void launch_stage(m2cx_solver* h, int vin, int vout, int mode, int phase 
   const int v = h->tile < 0 ? 0 : h->tile;
   hipEvent_t e0{};
   tic(h, name, &e0, st);
-  if (h->ustage && phase != 2)
-    (a.s.flux == M2CX_FLUX_HLLC ? ustage_launch_hllc : ustage_launch_other)(a, mode, v, st);
+  if (h->ustage && phase != 2) {
+    if (a.s.var_type != M2CX_VAR_PRIMITIVE) ustage_launch_gen(a, mode, st);
+    else (a.s.flux == M2CX_FLUX_HLLC ? ustage_launch_hllc : ustage_launch_other)(a, mode, v, st);
+  }
   a.phase = (h->ustage && phase == 0) ? 2 : phase;
   if (!h->ustage || phase == 2 || (phase == 0 && a.tflag)) launch_stage_variant(h, a, mode, v, st);
   toc(h, name, e0, st);

@@ -45,7 +45,7 @@ void stage_launch(const StageArgs& a, int mode, int variant, hipStream_t st) {
   }
 }
 
-void stage_launch_gen(const StageArgs& a, int mode, hipStream_t st) { launch<0, true>(a, mode, st); }
+void stage_launch_gen(const StageArgs& a, int mode, hipStream_t st) { launch<kGenTile, true>(a, mode, st); }
 
 void stage_launch_multi(const StageArgs* tab, const int* toff, int nm, int ntiles, int mode, int variant,
                         hipStream_t st) {

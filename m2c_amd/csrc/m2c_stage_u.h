@@ -1,26 +1,24 @@
 // The fused stage on tiles of one material (gfx950): the same stage as
 // stage_tile of m2c_stage.h, bit for bit, for tiles whose cells and the two
 // cells around them along each axis all hold one active material
-// (k_tile_mixed), with a primitive (or constant) reconstruction on a uniform
-// mesh and an HLLC, Roe or LLF flux.  That is nearly every tile of a run.
+// (k_tile_mixed), with linear reconstruction on a uniform mesh and an HLLC,
+// Roe or LLF flux.  That is nearly every tile of a run.
 #pragma once
 #include "m2c_exactdiv.h"
 #include "m2c_stage.h"
 
 namespace m2c {
 
-// Half the limited slopes of a cell with state v between the states vm and vp
-// along an axis, with the coefficients of a uniform mesh, A = B = 1 and (van
-// Albada) K = 2: lim_gmm and lim_va with the multiplications by one left out.
+// Limited slopes of a cell from the one-sided differences d0, d1 along an axis, with the coefficients of a uniform mesh, A = B = 1 and (van Albada)
+// K = 2: lim_gmm and lim_va with the multiplications by one left out.
 // The divisions of the five components are formed side by side, and not at
 // all where no lane of the wave has a slope to limit.
-__device__ __forceinline__ void half_slopes(const Scheme& s, const double* v, const double* vm, const double* vp,
-                                            double* h) {
+__device__ __forceinline__ void limited(const Scheme& s, const double* d0, const double* d1, double* h) {
   if (s.limiter == M2CX_LIM_VANALBADA) {
     bool z[5], any = false;
 #pragma unroll
     for (int p = 0; p < 5; p++) {
-      const double pr = (v[p] - vm[p]) * (vp[p] - v[p]);
+      const double pr = d0[p] * d1[p];
       z[p] = (pr <= 0) | (fabs(pr) < 1e-16);
       any |= !z[p];
       h[p] = 0.0;
@@ -32,29 +30,41 @@ __device__ __forceinline__ void half_slopes(const Scheme& s, const double* v, co
       bool ok = true;
 #pragma unroll
       for (int p = 0; p < 5; p++) {
-        const double d0 = v[p] - vm[p], d1 = vp[p] - v[p];
-        const double a = d0 * d0, b = d1 * d1, n = d1 * a + d0 * b;
-        const double r = 0.5 * Recip(a + b).quot(n);
+        const double a = d0[p] * d0[p], b = d1[p] * d1[p], n = d1[p] * a + d0[p] * b;
+        const double r = Recip(a + b).quot(n);
         ok &= z[p] | (a + b <= 0x1p600);
         h[p] = z[p] ? 0.0 : r;
       }
       if (!__all(ok)) {
 #pragma unroll
         for (int p = 0; p < 5; p++) {
-          const double d0 = v[p] - vm[p], d1 = vp[p] - v[p];
-          const double a = d0 * d0, b = d1 * d1;
-          const double r = 0.5 * ((d1 * a + d0 * b) / (a + b));
+          const double a = d0[p] * d0[p], b = d1[p] * d1[p];
+          const double r = (d1[p] * a + d0[p] * b) / (a + b);
           h[p] = z[p] ? 0.0 : r;
         }
       }
     }
   } else if (s.limiter == M2CX_LIM_GENERALIZED_MINMOD) {
 #pragma unroll
-    for (int p = 0; p < 5; p++) h[p] = 0.5 * lim_gmm(1.0, 1.0, s.gmm, v[p] - vm[p], vp[p] - v[p]);
+    for (int p = 0; p < 5; p++) h[p] = lim_gmm(1.0, 1.0, s.gmm, d0[p], d1[p]);
   } else {
 #pragma unroll
-    for (int p = 0; p < 5; p++) h[p] = 0.5 * (0.5 * ((v[p] - vm[p]) + (vp[p] - v[p])));
+    for (int p = 0; p < 5; p++) h[p] = 0.5 * (d0[p] + d1[p]);
   }
+}
+
+// half the slopes, from the cell's state v and its neighbours'
+__device__ __forceinline__ void half_slopes(const Scheme& s, const double* v, const double* vm, const double* vp,
+                                            double* h) {
+  double d0[5], d1[5];
+#pragma unroll
+  for (int p = 0; p < 5; p++) {
+    d0[p] = v[p] - vm[p];
+    d1[p] = vp[p] - v[p];
+  }
+  limited(s, d0, d1, h);
+#pragma unroll
+  for (int p = 0; p < 5; p++) h[p] *= 0.5;
 }
 
 // The cell value where a face state fails CheckState or would be clipped
@@ -75,13 +85,79 @@ __device__ __forceinline__ int keep_or_revert(const DevEos& E, const double* v, 
   return (bad ? 1 : 0) | ((bad & !clip) ? 2 : 0);
 }
 
+// The cell value q0 and half the limited slopes h of a cell along axis D in the
+// scheme's reconstruction variables (recon_slope; uniform mesh, one material;
+// x, y, z order).  v is the cell's state, vm and vp its neighbours'.
+__device__ __forceinline__ void slopes_in_vars(const DevEos& E, const Scheme& s, int D, const double* v,
+                                               const double* vm, const double* vp, double* q0, double* h) {
+  const int vtype = s.var_type;
+  const bool cons = (vtype == M2CX_VAR_CONSERVATIVE || vtype == M2CX_VAR_CONSERVATIVE_CHARACTERISTIC);
+  const bool chr = vtype != M2CX_VAR_CONSERVATIVE;
+  double d0[5], d1[5];
+  if (cons) {
+    double t[5];
+    eos_p2c(E, v, q0);
+    eos_p2c(E, vm, t);
+#pragma unroll
+    for (int p = 0; p < 5; p++) d0[p] = q0[p] - t[p];
+    eos_p2c(E, vp, t);
+#pragma unroll
+    for (int p = 0; p < 5; p++) d1[p] = t[p] - q0[p];
+  } else {
+#pragma unroll
+    for (int p = 0; p < 5; p++) {
+      q0[p] = v[p];
+      d0[p] = v[p] - vm[p];
+      d1[p] = vp[p] - v[p];
+    }
+  }
+  CharBasis b;
+  if (chr) {
+    char_setup(E, v, D, b);  // k_recon_flags reports c^2 < 0
+    double w[5];
+    if (cons) char_left(b, v, d0, w);
+    else char_from_prim(b, v, d0, w);
+#pragma unroll
+    for (int p = 0; p < 5; p++) d0[p] = w[p];
+    if (cons) char_left(b, v, d1, w);
+    else char_from_prim(b, v, d1, w);
+#pragma unroll
+    for (int p = 0; p < 5; p++) d1[p] = w[p];
+  }
+  limited(s, d0, d1, h);
+  if (chr) {
+    double w[5];
+    if (cons) char_right(b, v, h, w);
+    else char_to_prim(b, v, h, w);
+#pragma unroll
+    for (int p = 0; p < 5; p++) h[p] = w[p];
+  }
+#pragma unroll
+  for (int p = 0; p < 5; p++) h[p] *= 0.5;
+}
+// The minus or plus face (recon_face) of a cell whose six faces pass
+// CheckState; one that would be clipped reverts to the cell's state.
+__device__ __forceinline__ void face_in_vars(const DevEos& E, const Scheme& s, const double* v, const double* q0,
+                                             const double* h, bool minus, double* out) {
+  double u[5], f[5];
+#pragma unroll
+  for (int p = 0; p < 5; p++) u[p] = f[p] = minus ? q0[p] - h[p] : q0[p] + h[p];
+  if (s.var_type != M2CX_VAR_PRIMITIVE_CHARACTERISTIC) eos_c2p(E, u, f);
+  const bool clip = eos_would_clip(E, f);
+#pragma unroll
+  for (int p = 0; p < 5; p++) out[p] = clip ? v[p] : f[p];
+}
+
 // States along an axis: {rho, normal velocity, first and second tangential
 // velocity, p}, the tangential ones in x, y, z order.
 __device__ __forceinline__ void to_axis(int D, const double* v, double* w) {
+  // the empty asm keeps the selects from becoming an indexed load (see vsel)
+  double a = v[1], b = v[2], c = v[3];
+  asm("" : "+v"(a), "+v"(b), "+v"(c));
   w[0] = v[0];
-  w[1] = D == 0 ? v[1] : (D == 1 ? v[2] : v[3]);
-  w[2] = D == 0 ? v[2] : v[1];
-  w[3] = D == 2 ? v[2] : v[3];
+  w[1] = D == 0 ? a : (D == 1 ? b : c);
+  w[2] = D == 0 ? b : a;
+  w[3] = D == 2 ? b : c;
   w[4] = v[4];
 }
 // component of a state or flux array that holds entry q of the order above
@@ -273,8 +349,11 @@ __device__ __forceinline__ void ghost_axis(int bc, const CF5& V, long cg, int D,
 // cell and launch are 0.7 ms of a 256^3 launch).  256^3 water, RK3 launches:
 // 4.24 ms with stage_tile, 1.86 ms here (VALU issue on 64% of the cycles at
 // three waves per SIMD; held to 128 registers for four it spills: 2.88 ms);
-// 128x32x32 gas: 53 -> 24 us.
-template <int MODE, int BX, int BY, int BZ, bool HLLC>
+// 128x32x32 gas: 53 -> 24 us.  GEN (any reconstruction variables; a cell that
+// s.rflag marks is reconstructed in primitive ones): the slopes' eigenvectors
+// set the cost, formed once per cell and axis instead of for each of its two
+// faces (191x97x61 water, Roe, conservative-characteristic: 737 -> 330 us).
+template <int MODE, int BX, int BY, int BZ, bool HLLC, bool GEN>
 __device__ __forceinline__ void ustage_body(const StageArgs& a, int tile, const DevEos E,
                                             double (*sF)[TileShape<BX, BY, BZ>::NFACE]) {
   using TS = TileShape<BX, BY, BZ>;
@@ -306,15 +385,22 @@ __device__ __forceinline__ void ustage_body(const StageArgs& a, int tile, const 
       double vm[5], vp[5], h[5], l[5], r[5];
       load5(a.Vin, c - st, vm);
       load5(a.Vin, c + st, vp);
-      half_slopes(s, v, vm, vp, h);
+      if (GEN && !s.rflag[c]) {
+        double q0[5];
+        slopes_in_vars(E, s, D, v, vm, vp, q0, h);
+        face_in_vars(E, s, v, q0, h, true, l);
+        face_in_vars(E, s, v, q0, h, false, r);
+      } else {
+        half_slopes(s, v, vm, vp, h);
 #pragma unroll
-      for (int p = 0; p < 5; p++) {
-        l[p] = v[p] - h[p];
-        r[p] = v[p] + h[p];
+        for (int p = 0; p < 5; p++) {
+          l[p] = v[p] - h[p];
+          r[p] = v[p] + h[p];
+        }
+        const int bl = keep_or_revert(E, v, l), br = keep_or_revert(E, v, r);
+        fails |= ((bl & 1) | ((br & 1) << 1)) << (2 * D);
+        unf |= ((bl >> 1) | ((br >> 1) << 1)) << (2 * D);
       }
-      const int bl = keep_or_revert(E, v, l), br = keep_or_revert(E, v, r);
-      fails |= ((bl & 1) | ((br & 1) << 1)) << (2 * D);
-      unf |= ((bl >> 1) | ((br >> 1) << 1)) << (2 * D);
       const int slot = TS::slot(D, tx + (D == 0), ty + (D == 1), tz + (D == 2));
 #pragma unroll
       for (int p = 0; p < 5; p++) sF[p][slot] = r[p];
@@ -341,17 +427,27 @@ __device__ __forceinline__ void ustage_body(const StageArgs& a, int tile, const 
     if (fi < 0 || fj < 0 || fk < 0 || fi >= g.NX || fj >= g.NY || fk >= g.NZ) continue;
     const long cc = gidx(g, fi, fj, fk), st = axis_stride(g, D);
     double v[5], vm[5], vp[5], h[5], f[5];
+    if (GEN && !s.rflag[cc]) {
+      double q0[5], x[5];
+      load5(a.Vin, cc, v);
+      load5(a.Vin, cc - st, vm);
+      load5(a.Vin, cc + st, vp);
+      slopes_in_vars(E, s, D, v, vm, vp, q0, h);
+      face_in_vars(E, s, v, q0, h, plus, x);
+      to_axis(D, x, f);
+    } else {
 #pragma unroll
-    for (int p = 0; p < 5; p++) {
-      const int w = axis_comp(D, p);
-      v[p] = a.Vin(w, cc);
-      vm[p] = a.Vin(w, cc - st);
-      vp[p] = a.Vin(w, cc + st);
+      for (int p = 0; p < 5; p++) {
+        const int w = axis_comp(D, p);
+        v[p] = a.Vin(w, cc);
+        vm[p] = a.Vin(w, cc - st);
+        vp[p] = a.Vin(w, cc + st);
+      }
+      half_slopes(s, v, vm, vp, h);
+#pragma unroll
+      for (int p = 0; p < 5; p++) f[p] = plus ? v[p] - h[p] : v[p] + h[p];
+      keep_or_revert(E, v, f);
     }
-    half_slopes(s, v, vm, vp, h);
-#pragma unroll
-    for (int p = 0; p < 5; p++) f[p] = plus ? v[p] - h[p] : v[p] + h[p];
-    keep_or_revert(E, v, f);
     if (plus) {
 #pragma unroll
       for (int p = 0; p < 5; p++) lo[3][p] = f[p];
@@ -433,7 +529,7 @@ __device__ __forceinline__ void ustage_body(const StageArgs& a, int tile, const 
   stage_update<MODE>(a, E, in, i, j, k, c, r);
 }
 
-template <int MODE, int BX, int BY, int BZ, bool HLLC>
+template <int MODE, int BX, int BY, int BZ, bool HLLC, bool GEN>
 __device__ __forceinline__ void ustage_tile(const StageArgs& a, int tile) {
   __shared__ double sF[5][TileShape<BX, BY, BZ>::NFACE];
   if (a.tflag && a.tflag[tile]) return;
@@ -444,12 +540,12 @@ __device__ __forceinline__ void ustage_tile(const StageArgs& a, int tile) {
   const DevEos E = c_mats[a.s.mset].m[id];
   // one copy of the tile's code per type of equation of state, each without
   // the others' branches
-  if (E.type == M2CX_EOS_SG) ustage_body<MODE, BX, BY, BZ, HLLC>(a, tile, E, sF);
-  else if (E.type == M2CX_EOS_NASG) ustage_body<MODE, BX, BY, BZ, HLLC>(a, tile, E, sF);
-  else ustage_body<MODE, BX, BY, BZ, HLLC>(a, tile, E, sF);
+  if (E.type == M2CX_EOS_SG) ustage_body<MODE, BX, BY, BZ, HLLC, GEN>(a, tile, E, sF);
+  else if (E.type == M2CX_EOS_NASG) ustage_body<MODE, BX, BY, BZ, HLLC, GEN>(a, tile, E, sF);
+  else ustage_body<MODE, BX, BY, BZ, HLLC, GEN>(a, tile, E, sF);
 }
 
-template <int MODE, int BX, int BY, int BZ, bool HLLC>
+template <int MODE, int BX, int BY, int BZ, bool HLLC, bool GEN>
 __global__ void __launch_bounds__(BX * BY * BZ) k_stage_u(StageArgs a) {
   // read in place, as in k_stage
   const StageArgs& ar = *(const StageArgs*)__builtin_amdgcn_kernarg_segment_ptr();
@@ -457,18 +553,18 @@ __global__ void __launch_bounds__(BX * BY * BZ) k_stage_u(StageArgs a) {
   const int ntiles = ((g.NX + BX - 1) / BX) * ((g.NY + BY - 1) / BY) * ((g.NZ + BZ - 1) / BZ);
   const int tile = xcd_tile(ntiles);
   if (tile >= ntiles) return;
-  ustage_tile<MODE, BX, BY, BZ, HLLC>(ar, tile);
+  ustage_tile<MODE, BX, BY, BZ, HLLC, GEN>(ar, tile);
 }
 
 // the members of an ensemble in one launch, as k_stage_multi
-template <int MODE, int BX, int BY, int BZ, bool HLLC>
+template <int MODE, int BX, int BY, int BZ, bool HLLC, bool GEN>
 __global__ void __launch_bounds__(BX * BY * BZ) k_stage_u_multi(const StageArgs* __restrict__ tab,
                                                                  const int* __restrict__ toff, int nm) {
   const int total = toff[nm];
   const int t = xcd_tile(total);
   if (t >= total) return;
   const int m = multi_member(toff, nm, t);
-  ustage_tile<MODE, BX, BY, BZ, HLLC>(tab[m], t - toff[m]);
+  ustage_tile<MODE, BX, BY, BZ, HLLC, GEN>(tab[m], t - toff[m]);
 }
 
 }  // namespace m2c

@@ -16,12 +16,12 @@ static void launch(const StageArgs& a, int mode, hipStream_t st) {
   using T = Tile<V>;
   const dim3 grid = stage_grid(stage_tiles(a.g, T::X, T::Y, T::Z));
   switch (mode) {
-    case MODE_RESIDUAL: k_stage_u<MODE_RESIDUAL, T::X, T::Y, T::Z, HLLC><<<grid, T::NT, 0, st>>>(a); break;
-    case MODE_STAGE1: k_stage_u<MODE_STAGE1, T::X, T::Y, T::Z, HLLC><<<grid, T::NT, 0, st>>>(a); break;
-    case MODE_RK2_FINAL: k_stage_u<MODE_RK2_FINAL, T::X, T::Y, T::Z, HLLC><<<grid, T::NT, 0, st>>>(a); break;
-    case MODE_RK3_STAGE2: k_stage_u<MODE_RK3_STAGE2, T::X, T::Y, T::Z, HLLC><<<grid, T::NT, 0, st>>>(a); break;
-    case MODE_RK3_FINAL: k_stage_u<MODE_RK3_FINAL, T::X, T::Y, T::Z, HLLC><<<grid, T::NT, 0, st>>>(a); break;
-    case MODE_FE: k_stage_u<MODE_FE, T::X, T::Y, T::Z, HLLC><<<grid, T::NT, 0, st>>>(a); break;
+    case MODE_RESIDUAL: k_stage_u<MODE_RESIDUAL, T::X, T::Y, T::Z, HLLC, false><<<grid, T::NT, 0, st>>>(a); break;
+    case MODE_STAGE1: k_stage_u<MODE_STAGE1, T::X, T::Y, T::Z, HLLC, false><<<grid, T::NT, 0, st>>>(a); break;
+    case MODE_RK2_FINAL: k_stage_u<MODE_RK2_FINAL, T::X, T::Y, T::Z, HLLC, false><<<grid, T::NT, 0, st>>>(a); break;
+    case MODE_RK3_STAGE2: k_stage_u<MODE_RK3_STAGE2, T::X, T::Y, T::Z, HLLC, false><<<grid, T::NT, 0, st>>>(a); break;
+    case MODE_RK3_FINAL: k_stage_u<MODE_RK3_FINAL, T::X, T::Y, T::Z, HLLC, false><<<grid, T::NT, 0, st>>>(a); break;
+    case MODE_FE: k_stage_u<MODE_FE, T::X, T::Y, T::Z, HLLC, false><<<grid, T::NT, 0, st>>>(a); break;
   }
 }
 
@@ -30,10 +30,10 @@ static void launch_multi(const StageArgs* tab, const int* toff, int nm, int ntil
   using T = Tile<V>;
   const dim3 grid = stage_grid(ntiles);
   switch (mode) {
-    case MODE_STAGE1: k_stage_u_multi<MODE_STAGE1, T::X, T::Y, T::Z, HLLC><<<grid, T::NT, 0, st>>>(tab, toff, nm); break;
-    case MODE_RK2_FINAL: k_stage_u_multi<MODE_RK2_FINAL, T::X, T::Y, T::Z, HLLC><<<grid, T::NT, 0, st>>>(tab, toff, nm); break;
-    case MODE_RK3_STAGE2: k_stage_u_multi<MODE_RK3_STAGE2, T::X, T::Y, T::Z, HLLC><<<grid, T::NT, 0, st>>>(tab, toff, nm); break;
-    case MODE_RK3_FINAL: k_stage_u_multi<MODE_RK3_FINAL, T::X, T::Y, T::Z, HLLC><<<grid, T::NT, 0, st>>>(tab, toff, nm); break;
+    case MODE_STAGE1: k_stage_u_multi<MODE_STAGE1, T::X, T::Y, T::Z, HLLC, false><<<grid, T::NT, 0, st>>>(tab, toff, nm); break;
+    case MODE_RK2_FINAL: k_stage_u_multi<MODE_RK2_FINAL, T::X, T::Y, T::Z, HLLC, false><<<grid, T::NT, 0, st>>>(tab, toff, nm); break;
+    case MODE_RK3_STAGE2: k_stage_u_multi<MODE_RK3_STAGE2, T::X, T::Y, T::Z, HLLC, false><<<grid, T::NT, 0, st>>>(tab, toff, nm); break;
+    case MODE_RK3_FINAL: k_stage_u_multi<MODE_RK3_FINAL, T::X, T::Y, T::Z, HLLC, false><<<grid, T::NT, 0, st>>>(tab, toff, nm); break;
   }
 }
 

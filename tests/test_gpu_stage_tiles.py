@@ -75,6 +75,39 @@ def test_one_material(mat, flux, limiter, rough):
         _same_residual(gpu, o)
 
 
+VARS = [abi.VAR_CONSERVATIVE, abi.VAR_PRIMITIVE_CHARACTERISTIC, abi.VAR_CONSERVATIVE_CHARACTERISTIC]
+
+
+@pytest.mark.parametrize("mat", list(MATS))
+@pytest.mark.parametrize("var", VARS)
+@pytest.mark.parametrize("flux,limiter", [(abi.FLUX_HLLC, abi.LIM_VANALBADA), (abi.FLUX_ROE, abi.LIM_GMM),
+                                          (abi.FLUX_LLF, abi.LIM_NONE)])
+@pytest.mark.parametrize("rough", [False, True])
+def test_reconstruction_variables(mat, var, flux, limiter, rough):
+    """Rough states send some cells back to primitive variables, also cells
+    around a tile whose faces the tile forms."""
+    for n in ((35, 11, 9), (5, 3, 2)):
+        gpu, o = _pair(n, MATS[mat], _state(n, 6, rough), flux=flux, limiter=limiter, var_type=var)
+        _same_residual(gpu, o)
+
+
+@pytest.mark.parametrize("var", VARS)
+@pytest.mark.parametrize("overlap", [True, False])
+def test_reconstruction_variables_with_an_interface(var, overlap):
+    from m2c_amd import runtime
+    g, mats, nmat, s, V, ID, Phi = configs.c2_shock_bubble(32, radius=0.27)
+    s.var_type, s.flux, s.limiter = var, abi.FLUX_ROE, abi.LIM_GMM
+    o = ol.Oracle(g, mats, nmat, s)
+    o.set_state(V, ID, Phi)
+    gpu = runtime.Solver(g, mats, nmat, s)
+    gpu.set_overlap(overlap)
+    gpu.set_state(V, ID, Phi)
+    gpu.run_steps(3)
+    o.run_steps(3)
+    for a, b in zip(gpu.get_state(), o.get_state()):
+        assert np.array_equal(_inner(a), _inner(b))
+
+
 @pytest.mark.parametrize("n", [(1, 1, 1), (2, 1, 1), (1, 3, 1), (1, 1, 5), (33, 1, 1), (8, 8, 4), (9, 9, 5), (7, 65, 3)])
 @pytest.mark.parametrize("ti", [abi.TI_FE, abi.TI_RK2, abi.TI_RK3])
 def test_small_and_ragged_grids(n, ti):
