@@ -1932,8 +1932,10 @@ static int mlp_batch(m2cx_solver* h, const float* dX, const float* dT, const int
     c1 = 1.0f - std::pow(b1, (float)h->mlp.adam_t);
     c2 = 1.0f - std::pow(b2, (float)h->mlp.adam_t);
   }
-  k_mlp_adam<<<(MLP_NPAR + 255) / 256, 256, 0, h->stream>>>(h->mlp.theta, h->mlp.m, h->mlp.v, gpart, waves, lr, b1,
-                                                             b2, 1e-8f, c1, c2, gout, lpart, loss_acc);
+  const int blocks = (MLP_NPAR + 255) / 256, per = waves > MLP_DIRECT_WAVES ? mlp_rows_per_sum(waves) : 1;
+  if (per > 1) k_mlp_reduce<<<dim3(blocks, (waves + per - 1) / per), 256, 0, h->stream>>>(gpart, waves, per);
+  k_mlp_adam<<<blocks, 256, 0, h->stream>>>(h->mlp.theta, h->mlp.m, h->mlp.v, gpart, waves, per, lr, b1, b2, 1e-8f,
+                                            c1, c2, gout, lpart, loss_acc);
   if (lr > 0) k_mlp_refresh<<<16, 256, 0, h->stream>>>(h->mlp.theta, mlp_dev(h));
   HIPCHK(h, hipGetLastError());
   return 0;

@@ -19,6 +19,7 @@
 // copies are refreshed after every update.
 #pragma once
 #include <hip/hip_runtime.h>
+#include <algorithm>
 #include "m2c_kernels.h"
 
 namespace m2c {
@@ -385,20 +386,49 @@ __global__ void __launch_bounds__(64) k_mlp_train_step(MLPTrainArgs a) {
   }
 }
 
-// Sum of the partial gradients (fixed order, deterministic) and one Adam step
-// on the FP32 master parameters.
-__global__ void k_mlp_adam(float* theta, float* m, float* v, const float* gpart, int waves, float lr, float b1,
-                           float b2, float eps, float c1, float c2, float* gout, const float* lpart,
-                           double* loss_acc) {
+// Rows of partial gradients that one work-group of k_mlp_reduce adds up: at
+// least 8, and at most 64 sums are left for k_mlp_adam.
+__host__ inline int mlp_rows_per_sum(int waves) { return std::max(8, (waves + 63) / 64); }
+// waves above which the partial gradients are first summed in groups: up to
+// here k_mlp_adam's own loop over the rows takes no longer than a launch
+constexpr int MLP_DIRECT_WAVES = 16;
+
+// The partial gradients of rows [q per, (q + 1) per), q = blockIdx.y, summed in
+// order into the first of them (a fixed order: deterministic).  2 048 rows
+// (65 536 samples, 73 MB): added up by k_mlp_adam's 36 work-groups alone they
+// took 577 us, one load in flight per lane; 36 x 64 work-groups read them in
+// parallel (labels, loss and gradient of 65 536 problems: 1 326 -> 827 us).
+__global__ void __launch_bounds__(256) k_mlp_reduce(float* gpart, int waves, int per) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i == 0 && loss_acc) {
+  if (i >= MLP_NPAR) return;
+  const int w0 = blockIdx.y * per, w1 = min(waves, w0 + per);
+  float gsum = 0.0f;
+  for (int w = w0; w < w1; w++) gsum += gpart[(long)w * MLP_NPAR + i];
+  gpart[(long)w0 * MLP_NPAR + i] = gsum;
+}
+
+// Sum of the partial gradients (every `per`-th row; fixed order, deterministic)
+// and one Adam step on the FP32 master parameters; the first work-group also
+// adds up the squared errors, in double and in a fixed order.
+__global__ void __launch_bounds__(256) k_mlp_adam(float* theta, float* m, float* v, const float* gpart, int waves,
+                                                  int per, float lr, float b1, float b2, float eps, float c1, float c2,
+                                                  float* gout, const float* lpart, double* loss_acc) {
+  __shared__ double red[256];
+  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (blockIdx.x == 0 && loss_acc) {
     double sum = 0.0;
-    for (int w = 0; w < waves; w++) sum += lpart[w];
-    *loss_acc += sum;
+    for (int w = threadIdx.x; w < waves; w += 256) sum += lpart[w];
+    red[threadIdx.x] = sum;
+    __syncthreads();
+    for (int o = 128; o > 0; o >>= 1) {
+      if (threadIdx.x < o) red[threadIdx.x] += red[threadIdx.x + o];
+      __syncthreads();
+    }
+    if (threadIdx.x == 0) *loss_acc += red[0];
   }
   if (i >= MLP_NPAR) return;
   float gsum = 0.0f;
-  for (int w = 0; w < waves; w++) gsum += gpart[(long)w * MLP_NPAR + i];
+  for (int w = 0; w < waves; w += per) gsum += gpart[(long)w * MLP_NPAR + i];
   if (gout) gout[i] = gsum;
   if (lr <= 0.0f) return;
   const float mi = b1 * m[i] + (1.0f - b1) * gsum;

@@ -65,6 +65,34 @@ def test_training_gradient_matches_oracle():
         assert r <= 5e-2, (name, r)
 
 
+@pytest.mark.parametrize("n", [31, 32, 512, 513, 1024, 2047, 16384, 16385, 16416, 65536])
+def test_gradient_is_the_sum_over_parts(n):
+    """The partial gradients of all waves against those of parts that one loop
+    adds up (512 samples).  Where n / 512 is a power of two the parts' bf16
+    products are the same ones scaled, and only the FP32 sums' order differs:
+    at most 96 additions of terms whose sizes add up to at most
+    sqrt(2048) = 45 times the sum's, 96 * 2^-24 * 45 < 3e-4.  Elsewhere the scale
+    1/n enters the bf16 roundings, 2^-9 each, of two products.  A row of
+    2048 left out changes the sum by 1/45."""
+    sol, _ = _solver()
+    rng = np.random.default_rng(n)
+    theta = mlp_ref.init_params(7)
+    theta[4736 + 4096:4736 + 4160] = rng.normal(0, 0.1, 64)
+    sol.mlp_set_params(theta)
+    X = rng.normal(size=(n, 8)).astype(np.float32)
+    T = rng.normal(size=n).astype(np.float32)
+    loss, g = sol.mlp_loss_grad(X, T)
+    gs, ls = np.zeros(g.size), 0.0
+    for a in range(0, n, 512):
+        x, t = X[a:a + 512], T[a:a + 512]
+        l1, g1 = sol.mlp_loss_grad(x, t)
+        gs += g1.astype(np.float64) * (len(t) / n)
+        ls += float(l1) * len(t) / n
+    exact = n < 512 or (n % 512 == 0 and (n // 512) & (n // 512 - 1) == 0)
+    assert np.linalg.norm(g - gs) <= (3e-4 if exact else 2.0**-8) * np.linalg.norm(gs)
+    assert abs(loss - ls) <= 1e-6 * ls
+
+
 def _air_pair():
     return abi.materials(abi.material("SG", gamma=1.4), abi.material("SG", gamma=1.4))
 
