@@ -75,10 +75,10 @@ struct m2cx_solver {
   // multi-material
   MPBuffers mp{};
   bool multimat = false;
-  // the stage kernel's non-interface tiles run on stream2 while the
-  // interface Riemann problems are solved on stream (fork / join events)
+  // the one-material stage tiles and the stage's level set run on stream2 while
+  // the interface Riemann problems are solved on stream (fork / join events)
   hipStream_t stream2 = nullptr;
-  hipEvent_t ev_fork = nullptr, ev_join = nullptr;
+  hipEvent_t ev_fork = nullptr, ev_riem = nullptr, ev_join = nullptr;
   bool overlap = false;
   // stage tiles: tflag marks the mixed ones (k_tile_mixed, once per step);
   // the others run the one-material kernel when the scheme has one (ustage).
@@ -628,6 +628,7 @@ static int create_impl(const m2cx_grid* grid, const m2cx_material* mats, int nma
     if (!getenv("M2C_NO_OVERLAP")) {
       HIPCHK(h, hipStreamCreateWithFlags(&h->stream2, hipStreamNonBlocking));
       HIPCHK(h, hipEventCreateWithFlags(&h->ev_fork, hipEventDisableTiming));
+      HIPCHK(h, hipEventCreateWithFlags(&h->ev_riem, hipEventDisableTiming));
       HIPCHK(h, hipEventCreateWithFlags(&h->ev_join, hipEventDisableTiming));
       h->overlap = true;
     }
@@ -672,6 +673,7 @@ int m2cx_destroy(m2cx_solver* h) {
   if (h->tflag) hipFree(h->tflag);
   if (h->stream2) hipStreamSynchronize(h->stream2);
   if (h->ev_fork) hipEventDestroy(h->ev_fork);
+  if (h->ev_riem) hipEventDestroy(h->ev_riem);
   if (h->ev_join) hipEventDestroy(h->ev_join);
   if (h->stream2) hipStreamDestroy(h->stream2);
   mat_slot_release(h);
@@ -978,39 +980,40 @@ static void interface_stage(m2cx_solver* h, int vin, int stage1) {
 // the level-set residual in the band, then (which >= 0) the RK combination
 // on its useful nodes inside the domain and the boundary fill of the field
 // it wrote (LevelSetOperator.cpp:880-955, 152-196, 408-508)
-static void levelset_band(m2cx_solver* h, CF5 V, int which) {
+static void levelset_band(m2cx_solver* h, CF5 V, int which, hipStream_t st) {
   MPBuffers& B = h->mp;
   const int LB = nb_blocks(h);
   LSArgs a = mp_ls_args(B, h->g, V, which, h->cnt);
   if (B.fv.on) {
     const long nf = 2L * ((long)h->g.NY * h->g.NZ + (long)h->g.NX * h->g.NZ + (long)h->g.NX * h->g.NY);
-    k_nb_fv_recon<<<LB, 256, 0, h->stream>>>(a, h->nb);
-    k_nb_fv_ghost<<<blocks_for(nf), 256, 0, h->stream>>>(a, h->nb);
-    k_nb_fv_flux<<<LB, 256, 0, h->stream>>>(a, h->nb);
+    k_nb_fv_recon<<<LB, 256, 0, st>>>(a, h->nb);
+    k_nb_fv_ghost<<<blocks_for(nf), 256, 0, st>>>(a, h->nb);
+    k_nb_fv_flux<<<LB, 256, 0, st>>>(a, h->nb);
   } else {
-    k_nb_ls_residual<<<LB, 256, 0, h->stream>>>(a, h->nb);
+    k_nb_ls_residual<<<LB, 256, 0, st>>>(a, h->nb);
   }
   if (which < 0) return;
-  k_nb_ls_combine<<<LB, 256, 0, h->stream>>>(h->g, h->nb, which, B.phi, B.phi1, B.rls, h->cnt);
+  k_nb_ls_combine<<<LB, 256, 0, st>>>(h->g, h->nb, which, B.phi, B.phi1, B.rls, h->cnt);
   double* tgt = (which == 1 || which == 3) ? B.phi1 : B.phi;
   const long nf = 2L * ((long)h->g.NY * h->g.NZ + (long)h->g.NX * h->g.NZ + (long)h->g.NX * h->g.NY);
-  k_ls_bc<<<blocks_for(nf), 256, 0, h->stream>>>(h->g, tgt, B.lsbc[0], B.lsbc[1], B.lsbc[2], B.lsbc[3], B.lsbc[4],
+  k_ls_bc<<<blocks_for(nf), 256, 0, st>>>(h->g, tgt, B.lsbc[0], B.lsbc[1], B.lsbc[2], B.lsbc[3], B.lsbc[4],
                                                 B.lsbc[5]);
 }
 
-static void levelset_stage(m2cx_solver* h, int vin, int which) {
+static void levelset_stage(m2cx_solver* h, int vin, int which, hipStream_t st = nullptr) {
   if (!h->multimat || h->nls == 0) return;
+  if (!st) st = h->stream;
   hipEvent_t e0{};
-  tic(h, "levelset", &e0);
+  tic(h, "levelset", &e0, st);
   for (int q = 0; q < h->nls; q++) {
     swap_ls(h, q);
     if (h->nb.bw)
-      levelset_band(h, cf5(h, h->V[vin]), which);
+      levelset_band(h, cf5(h, h->V[vin]), which, st);
     else
-      mp_levelset(h->mp, h->g, cf5(h, h->V[vin]), which, h->cnt, h->stream);
+      mp_levelset(h->mp, h->g, cf5(h, h->V[vin]), which, h->cnt, st);
     swap_ls(h, q);
   }
-  toc(h, "levelset", e0);
+  toc(h, "levelset", e0, st);
 }
 
 int m2cx_compute_residual(m2cx_solver* h, int v_field, int capture_riemann) {
@@ -1082,6 +1085,10 @@ static int stage_specs(int ti, StageSpec* out) {
   out[2] = StageSpec{2, 0, MODE_RK3_FINAL, 0, 0, 4};
   return 3;
 }
+
+// the level-set stages that write Phi in place (the last of RK2 and RK3); the
+// others write a field that nothing else of the stage reads
+static bool writes_phi(int ls_which) { return ls_which == 2 || ls_which == 4; }
 
 // the part of a stage after its interface Riemann problems
 static void stage_after_riemann(m2cx_solver* h, const StageSpec& sp) {
@@ -1511,15 +1518,23 @@ static void split_stage(m2cx_solver* h, const StageSpec& sp) {
   tic(h, "riemann", &e0);
   mp_riemann(h->mp, h->g, h->s, cf5(h, h->V[sp.vin]), h->ID, sp.stage1, h->cnt, h->stream);
   toc(h, "riemann", e0);
+  hipEventRecord(h->ev_riem, h->stream);
   hipStreamWaitEvent(h->stream2, h->ev_fork, 0);
   launch_stage(h, sp.vin, sp.vout, sp.mode, 1);
+  // the stage's level set follows on stream2, where it is hidden behind the
+  // Riemann launch and the mixed tiles (a 200-cell tube: two launches, 9 us of
+  // a 78 us stage; 512x256x256: 0.8 of 12 ms).  It reads the stage's input alone;
+  // the final stage writes Phi, from which the Riemann launch takes the
+  // interface normals, and waits for that launch
+  const bool ls2 = sp.ls_which >= 0;
+  if (ls2 && writes_phi(sp.ls_which)) hipStreamWaitEvent(h->stream2, h->ev_riem, 0);
+  if (ls2) levelset_stage(h, sp.vin, sp.ls_which, h->stream2);
   hipEventRecord(h->ev_join, h->stream2);
   launch_stage(h, sp.vin, sp.vout, sp.mode, 2);
   hipStreamWaitEvent(h->stream, h->ev_join, 0);
   if (sp.resync)
     k_resync<<<grid_blocks(nin), 256, 0, h->stream>>>(h->g, h->s.mset, cf5(h, h->V[sp.vout]), f5(h, h->U1), h->ID,
                                                        h->cnt);
-  if (sp.ls_which >= 0) levelset_stage(h, sp.vin, sp.ls_which);
 }
 
 // One TimeIntegrator step with dt already in cnt->dt (TimeIntegrator.cpp:167-715)
@@ -2019,7 +2034,7 @@ int m2cx_levelset_residual(m2cx_solver* h, int v_field) {
     swap_ls(h, q);
     const bool unbuilt = h->nb.bw && !h->nb.built;
     if (!unbuilt && h->nb.bw)
-      levelset_band(h, cf5(h, h->V[v_field]), -1);
+      levelset_band(h, cf5(h, h->V[v_field]), -1, h->stream);
     else if (!unbuilt)
       mp_levelset(h->mp, h->g, cf5(h, h->V[v_field]), -1, h->cnt, h->stream);
     swap_ls(h, q);
@@ -2065,7 +2080,7 @@ struct m2cx_ensemble {
   // batched Riemann launch runs on stream
   bool overlap = false;
   hipStream_t stream2 = nullptr;
-  hipEvent_t ev_fork = nullptr, ev_join = nullptr;
+  hipEvent_t ev_fork = nullptr, ev_riem = nullptr, ev_join = nullptr;
   // the stage kernel of all split members that share a tile shape, one
   // launch per stage and phase (k_stage_multi): member tables [stage][phase]
   // and tile-count prefix sums
@@ -2148,12 +2163,17 @@ static void ensemble_step(m2cx_ensemble* e) {
       k_riem_count<<<e->nriem, 256, 0, e->stream>>>(e->dmem[q]);
     }
     if (e->overlap) {
+      hipEventRecord(e->ev_riem, e->stream);
       // the stage tiles of all members: one launch per tile shape, tiles
       // without interface faces beside the Riemann launch, the others after it
       hipStreamWaitEvent(e->stream2, e->ev_fork, 0);
       for (const auto& c : e->classes) launch_class(c, q, 1, sp[q].mode, e->stream2);
       for (m2cx_solver* h : act)
         if (split(h) && !e->classed.count(h)) launch_stage(h, sp[q].vin, sp[q].vout, sp[q].mode, 1);
+      // the level sets of split members, as in split_stage
+      if (writes_phi(sp[q].ls_which)) hipStreamWaitEvent(e->stream2, e->ev_riem, 0);
+      for (m2cx_solver* h : act)
+        if (split(h)) levelset_stage(h, sp[q].vin, sp[q].ls_which, e->stream2);
       hipEventRecord(e->ev_join, e->stream2);
       for (const auto& c : e->classes) launch_class(c, q, 2, sp[q].mode, e->stream);
       for (m2cx_solver* h : act)
@@ -2171,7 +2191,6 @@ static void ensemble_step(m2cx_ensemble* e) {
       if (sp[q].resync)
         k_resync<<<grid_blocks(nin), 256, 0, h->stream>>>(h->g, h->s.mset, cf5(h, h->V[sp[q].vout]), f5(h, h->U1),
                                                            h->ID, h->cnt);
-      if (sp[q].ls_which >= 0) levelset_stage(h, sp[q].vin, sp[q].ls_which);
     }
   }
   for (m2cx_solver* h : act)
@@ -2346,6 +2365,7 @@ int m2cx_ensemble_create(m2cx_solver* const* members, int n, m2cx_ensemble** out
   if (e->overlap) {
     EHIPCHK(e, hipStreamCreateWithFlags(&e->stream2, hipStreamNonBlocking));
     EHIPCHK(e, hipEventCreateWithFlags(&e->ev_fork, hipEventDisableTiming));
+    EHIPCHK(e, hipEventCreateWithFlags(&e->ev_riem, hipEventDisableTiming));
     EHIPCHK(e, hipEventCreateWithFlags(&e->ev_join, hipEventDisableTiming));
   }
   return ensemble_build(e);
@@ -2419,6 +2439,7 @@ int m2cx_ensemble_destroy(m2cx_ensemble* e) {
   hipFree(e->slab);
   free_classes(e);
   if (e->ev_fork) hipEventDestroy(e->ev_fork);
+  if (e->ev_riem) hipEventDestroy(e->ev_riem);
   if (e->ev_join) hipEventDestroy(e->ev_join);
   if (e->stream2) hipStreamDestroy(e->stream2);
   if (e->stream) hipStreamDestroy(e->stream);
