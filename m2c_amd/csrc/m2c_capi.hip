@@ -954,8 +954,17 @@ static void guess_stage(m2cx_solver* h, int vin) {
 // with Flux = Godunov the exact-solver fluxes of the single-material faces.
 static void recon_stage(m2cx_solver* h, int vin) {
   const long nin = (long)h->g.NX * h->g.NY * h->g.NZ;
-  if (h->rflag)
-    k_recon_flags<<<grid_blocks(nin), 256, 0, h->stream>>>(h->g, h->s, cf5(h, h->V[vin]), h->ID, h->rflag, h->cnt);
+  if (h->rflag) {
+    // where the one-material stage kernel runs, its tiles' cells are marked by
+    // code for one material and the others by the general code
+    const bool u = h->ustage, rest = !u || needs_tflags(h);
+    int tx, ty, tz;
+    stage_tile_dims(h, tx, ty, tz);
+    if (u) recon_flags_launch_u(stage_args(h, vin, -1, MODE_RESIDUAL), h->rflag, h->stream);
+    if (rest)
+      k_recon_flags<<<grid_blocks(nin), 256, 0, h->stream>>>(h->g, h->s, cf5(h, h->V[vin]), h->ID, h->rflag, h->cnt,
+                                                             u ? h->tflag : nullptr, tx, ty, tz);
+  }
   if (h->gflux) {
     hipEvent_t e0{};
     tic(h, "godunov", &e0);

@@ -11,12 +11,14 @@ namespace m2c {
 // instead (Reconstructor.cpp:722-778).  c0^2 < 0 in a characteristic
 // transform is the reference's abort (FluxFcnBase.h:315-320).
 __global__ void k_recon_flags(DevGrid g, Scheme s, CF5 V, const unsigned char* __restrict__ ID,
-                              unsigned char* __restrict__ flag, DevCounters* cnt) {
+                              unsigned char* __restrict__ flag, DevCounters* cnt,
+                              const unsigned char* __restrict__ mixed, int BX, int BY, int BZ) {
   const DevMats& M = c_mats[s.mset];
   const long n = (long)g.NX * g.NY * g.NZ;
   for (long q = blockIdx.x * (long)blockDim.x + threadIdx.x; q < n; q += (long)gridDim.x * blockDim.x) {
     int i, j, k;
     cell_ijk(g, q, i, j, k);
+    if (mixed && !mixed[i / BX + ((g.NX + BX - 1) / BX) * (j / BY + ((g.NY + BY - 1) / BY) * (k / BZ))]) continue;
     const long c = gidx(g, i, j, k);
     const int myid = ID[c];
     if (myid == s.inactive) {

@@ -42,6 +42,8 @@ void ustage_launch_multi_other(const StageArgs* tab, const int* toff, int nm, in
                                hipStream_t st);
 // reconstruction in conservative or characteristic variables
 void ustage_launch_gen(const StageArgs& a, int mode, hipStream_t st);
+// the marks of k_recon_flags on the tiles of one material
+void recon_flags_launch_u(const StageArgs& a, unsigned char* flag, hipStream_t st);
 hipError_t ustage_set_materials_gen(int slot, const DevMats& m);
 hipError_t ustage_set_materials_hllc(int slot, const DevMats& m);
 hipError_t ustage_set_materials_other(int slot, const DevMats& m);

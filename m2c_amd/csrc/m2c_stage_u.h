@@ -87,8 +87,9 @@ __device__ __forceinline__ int keep_or_revert(const DevEos& E, const double* v, 
 
 // The cell value q0 and half the limited slopes h of a cell along axis D in the
 // scheme's reconstruction variables (recon_slope; uniform mesh, one material;
-// x, y, z order).  v is the cell's state, vm and vp its neighbours'.
-__device__ __forceinline__ void slopes_in_vars(const DevEos& E, const Scheme& s, int D, const double* v,
+// x, y, z order).  v is the cell's state, vm and vp its neighbours'.  Returns
+// whether the eigenvectors exist (c^2 >= 0).
+__device__ __forceinline__ bool slopes_in_vars(const DevEos& E, const Scheme& s, int D, const double* v,
                                                const double* vm, const double* vp, double* q0, double* h) {
   const int vtype = s.var_type;
   const bool cons = (vtype == M2CX_VAR_CONSERVATIVE || vtype == M2CX_VAR_CONSERVATIVE_CHARACTERISTIC);
@@ -112,8 +113,9 @@ __device__ __forceinline__ void slopes_in_vars(const DevEos& E, const Scheme& s,
     }
   }
   CharBasis b;
+  bool ok = true;
   if (chr) {
-    char_setup(E, v, D, b);  // k_recon_flags reports c^2 < 0
+    ok = char_setup(E, v, D, b);
     double w[5];
     if (cons) char_left(b, v, d0, w);
     else char_from_prim(b, v, d0, w);
@@ -134,15 +136,22 @@ __device__ __forceinline__ void slopes_in_vars(const DevEos& E, const Scheme& s,
   }
 #pragma unroll
   for (int p = 0; p < 5; p++) h[p] *= 0.5;
+  return ok;
 }
-// The minus or plus face (recon_face) of a cell whose six faces pass
-// CheckState; one that would be clipped reverts to the cell's state.
-__device__ __forceinline__ void face_in_vars(const DevEos& E, const Scheme& s, const double* v, const double* q0,
-                                             const double* h, bool minus, double* out) {
-  double u[5], f[5];
+// the minus or plus face itself (recon_face)
+__device__ __forceinline__ void face_from_vars(const DevEos& E, const Scheme& s, const double* q0, const double* h,
+                                               bool minus, double* f) {
+  double u[5];
 #pragma unroll
   for (int p = 0; p < 5; p++) u[p] = f[p] = minus ? q0[p] - h[p] : q0[p] + h[p];
   if (s.var_type != M2CX_VAR_PRIMITIVE_CHARACTERISTIC) eos_c2p(E, u, f);
+}
+// The minus or plus face of a cell whose six faces pass CheckState (it is not
+// in s.rflag); one that would be clipped reverts to the cell's state.
+__device__ __forceinline__ void face_in_vars(const DevEos& E, const Scheme& s, const double* v, const double* q0,
+                                             const double* h, bool minus, double* out) {
+  double f[5];
+  face_from_vars(E, s, q0, h, minus, f);
   const bool clip = eos_would_clip(E, f);
 #pragma unroll
   for (int p = 0; p < 5; p++) out[p] = clip ? v[p] : f[p];

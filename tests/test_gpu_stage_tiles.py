@@ -140,6 +140,19 @@ def test_inactive_cells_in_a_one_material_solver():
         assert np.array_equal(_g[live], _o[live]), v
 
 
+@pytest.mark.parametrize("var", VARS)
+def test_inactive_cells_in_other_variables(var):
+    n = (40, 18, 13)
+    V = _state(n, 8, True)
+    gpu, o = _pair(n, MATS["stiff"], V, var_type=var)
+    ID = np.zeros(V.shape[:3], dtype=np.int32)
+    ID[5:8, 7:9, 20:23] = 1
+    gpu.upload(abi.FIELD_ID, ID)
+    o.set_state(V, ID, None)
+    live = _inner(ID) == 0
+    assert np.array_equal(_inner(gpu.compute_residual())[live], _inner(o.residual())[live])
+
+
 @pytest.mark.parametrize("case", ["denormal", "tiny", "huge", "vacuum", "zeros"])
 def test_ends_of_the_fast_range(case):
     """Velocities down to denormals (a wave's exponential front), states far
