@@ -1508,11 +1508,15 @@ static int end_of_step(m2cx_solver* h) {
   return 0;
 }
 
-// One stage with the stage kernel's tiles that touch no interface face
-// running on stream2 while the interface Riemann problems are solved: they
-// read V_in and write V_out (different fields) and no interface flux.  The
-// tiles with interface faces follow the Riemann launch; the level set waits
-// for both.  Results are those of the single launch (same code per tile).
+// Cells from which the last stage's level set, which waits for the Riemann
+// launch, runs on stream2: below, that wait costs more than the two launches it
+// hides (a 200-cell tube lost 2.9 % to the event alone; 512x256x256 gains 1.6 %).
+constexpr long LS_BESIDE_CELLS = 1L << 20;
+
+// One stage with the tiles of one material running on stream2 while the
+// interface Riemann problems are solved: they read V_in and write V_out
+// (different fields) and no interface flux.  The mixed tiles follow the
+// Riemann launch.  Results are those of the single launch (same code per tile).
 static void split_stage(m2cx_solver* h, const StageSpec& sp) {
   const long nin = (long)h->g.NX * h->g.NY * h->g.NZ;
   fill_iface_ls(h);
@@ -1527,16 +1531,16 @@ static void split_stage(m2cx_solver* h, const StageSpec& sp) {
   tic(h, "riemann", &e0);
   mp_riemann(h->mp, h->g, h->s, cf5(h, h->V[sp.vin]), h->ID, sp.stage1, h->cnt, h->stream);
   toc(h, "riemann", e0);
-  hipEventRecord(h->ev_riem, h->stream);
+  // The stage's level set follows the tiles of one material on stream2, hidden
+  // behind the Riemann launch and the mixed tiles.  It reads the stage's input
+  // alone; the final stage writes Phi, from which the Riemann launch takes the
+  // interface normals, and has to wait for that launch.
+  const bool after = writes_phi(sp.ls_which);
+  const bool ls2 = sp.ls_which >= 0 && (!after || nin >= LS_BESIDE_CELLS);
+  if (ls2 && after) hipEventRecord(h->ev_riem, h->stream);
   hipStreamWaitEvent(h->stream2, h->ev_fork, 0);
   launch_stage(h, sp.vin, sp.vout, sp.mode, 1);
-  // the stage's level set follows on stream2, where it is hidden behind the
-  // Riemann launch and the mixed tiles (a 200-cell tube: two launches, 9 us of
-  // a 78 us stage; 512x256x256: 0.8 of 12 ms).  It reads the stage's input alone;
-  // the final stage writes Phi, from which the Riemann launch takes the
-  // interface normals, and waits for that launch
-  const bool ls2 = sp.ls_which >= 0;
-  if (ls2 && writes_phi(sp.ls_which)) hipStreamWaitEvent(h->stream2, h->ev_riem, 0);
+  if (ls2 && after) hipStreamWaitEvent(h->stream2, h->ev_riem, 0);
   if (ls2) levelset_stage(h, sp.vin, sp.ls_which, h->stream2);
   hipEventRecord(h->ev_join, h->stream2);
   launch_stage(h, sp.vin, sp.vout, sp.mode, 2);
@@ -1544,6 +1548,7 @@ static void split_stage(m2cx_solver* h, const StageSpec& sp) {
   if (sp.resync)
     k_resync<<<grid_blocks(nin), 256, 0, h->stream>>>(h->g, h->s.mset, cf5(h, h->V[sp.vout]), f5(h, h->U1), h->ID,
                                                        h->cnt);
+  if (sp.ls_which >= 0 && !ls2) levelset_stage(h, sp.vin, sp.ls_which);
 }
 
 // One TimeIntegrator step with dt already in cnt->dt (TimeIntegrator.cpp:167-715)
@@ -2089,7 +2094,7 @@ struct m2cx_ensemble {
   // batched Riemann launch runs on stream
   bool overlap = false;
   hipStream_t stream2 = nullptr;
-  hipEvent_t ev_fork = nullptr, ev_riem = nullptr, ev_join = nullptr;
+  hipEvent_t ev_fork = nullptr, ev_join = nullptr;
   // the stage kernel of all split members that share a tile shape, one
   // launch per stage and phase (k_stage_multi): member tables [stage][phase]
   // and tile-count prefix sums
@@ -2172,17 +2177,12 @@ static void ensemble_step(m2cx_ensemble* e) {
       k_riem_count<<<e->nriem, 256, 0, e->stream>>>(e->dmem[q]);
     }
     if (e->overlap) {
-      hipEventRecord(e->ev_riem, e->stream);
       // the stage tiles of all members: one launch per tile shape, tiles
       // without interface faces beside the Riemann launch, the others after it
       hipStreamWaitEvent(e->stream2, e->ev_fork, 0);
       for (const auto& c : e->classes) launch_class(c, q, 1, sp[q].mode, e->stream2);
       for (m2cx_solver* h : act)
         if (split(h) && !e->classed.count(h)) launch_stage(h, sp[q].vin, sp[q].vout, sp[q].mode, 1);
-      // the level sets of split members, as in split_stage
-      if (writes_phi(sp[q].ls_which)) hipStreamWaitEvent(e->stream2, e->ev_riem, 0);
-      for (m2cx_solver* h : act)
-        if (split(h)) levelset_stage(h, sp[q].vin, sp[q].ls_which, e->stream2);
       hipEventRecord(e->ev_join, e->stream2);
       for (const auto& c : e->classes) launch_class(c, q, 2, sp[q].mode, e->stream);
       for (m2cx_solver* h : act)
@@ -2200,6 +2200,7 @@ static void ensemble_step(m2cx_ensemble* e) {
       if (sp[q].resync)
         k_resync<<<grid_blocks(nin), 256, 0, h->stream>>>(h->g, h->s.mset, cf5(h, h->V[sp[q].vout]), f5(h, h->U1),
                                                            h->ID, h->cnt);
+      if (sp[q].ls_which >= 0) levelset_stage(h, sp[q].vin, sp[q].ls_which);
     }
   }
   for (m2cx_solver* h : act)
@@ -2374,7 +2375,6 @@ int m2cx_ensemble_create(m2cx_solver* const* members, int n, m2cx_ensemble** out
   if (e->overlap) {
     EHIPCHK(e, hipStreamCreateWithFlags(&e->stream2, hipStreamNonBlocking));
     EHIPCHK(e, hipEventCreateWithFlags(&e->ev_fork, hipEventDisableTiming));
-    EHIPCHK(e, hipEventCreateWithFlags(&e->ev_riem, hipEventDisableTiming));
     EHIPCHK(e, hipEventCreateWithFlags(&e->ev_join, hipEventDisableTiming));
   }
   return ensemble_build(e);
@@ -2448,7 +2448,6 @@ int m2cx_ensemble_destroy(m2cx_ensemble* e) {
   hipFree(e->slab);
   free_classes(e);
   if (e->ev_fork) hipEventDestroy(e->ev_fork);
-  if (e->ev_riem) hipEventDestroy(e->ev_riem);
   if (e->ev_join) hipEventDestroy(e->ev_join);
   if (e->stream2) hipStreamDestroy(e->stream2);
   if (e->stream) hipStreamDestroy(e->stream);

@@ -207,3 +207,27 @@ def test_mixed_and_one_material_tiles(water, variant):
         Vg, IDg, Pg = gpu.get_state()
         assert np.array_equal(_inner(IDg), _inner(IDo)) and np.array_equal(_inner(Pg), _inner(Po))
         assert np.array_equal(_inner(Vg), _inner(Vo)), np.abs(_inner(Vg) - _inner(Vo)).max()
+
+
+@pytest.mark.parametrize("integrator", [abi.TI_RK2, abi.TI_RK3])
+@pytest.mark.parametrize("bandwidth", [None, 8])
+def test_level_set_beside_the_riemann_launch(integrator, bandwidth):
+    """Grids of 2^20 cells and more: the level set on the second stream, against
+    the run on one stream."""
+    from m2c_amd import runtime
+    g, mats, nmat, s, V, ID, Phi = configs.c2_shock_bubble(102)
+    s.integrator = integrator
+    if bandwidth:
+        s.ls_bandwidth = bandwidth
+        s.reinit_frequency = 1
+    out = []
+    for overlap in (True, False):
+        gpu = runtime.Solver(g, mats, nmat, s)
+        gpu.set_overlap(overlap)
+        gpu.set_state(V, ID, Phi)
+        if bandwidth:
+            gpu.construct_narrow_band()
+        gpu.run_steps(2)
+        out.append([np.array(a) for a in gpu.get_state()])
+    for a, b in zip(*out):
+        assert np.array_equal(_inner(a), _inner(b))
