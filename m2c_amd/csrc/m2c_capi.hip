@@ -1756,7 +1756,7 @@ int m2cx_riemann_batch_noalloc(m2cx_solver* h, int n, const double* dir, const d
     k_mlp_compose<<<(n + 255) / 256, 256, 0, h->stream>>>(n, y, P, pc, ok, dguess);
   }
   const MPBuffers& B = h->mp;
-  k_riemann_batch<<<(NOALLOC_LANES + 127) / 128, 128, 0, h->stream>>>(
+  k_riemann_batch<<<NOALLOC_LANES / 64, 64, 0, h->stream>>>(
       h->s.mset, B.rc, n, dir, Vm, idm, Vp, idp, Vs, id, Vsm, Vsp, err, it, fe, slab, NOALLOC_LANES, NOALLOC_PATHCAP,
       dguess, h->cnt);
   HIPCHK(h, hipGetLastError());
@@ -1834,7 +1834,7 @@ int m2cx_riemann_batch(m2cx_solver* h, int n, const double* dir, const double* V
     hipFree(X); hipFree(y); hipFree(P); hipFree(pc); hipFree(ok);
   }
   MPBuffers& B = h->mp;
-  k_riemann_batch<<<(B.lanes + 127) / 128, 128, 0, h->stream>>>(h->s.mset, B.rc, n, dd, dVm, didm, dVp, didp, dVs, did, dVsm,
+  k_riemann_batch<<<B.lanes / 64, 64, 0, h->stream>>>(h->s.mset, B.rc, n, dd, dVm, didm, dVp, didp, dVs, did, dVsm,
                                                                  dVsp, derr, dit, dfe, B.slab, B.lanes, B.pathcap,
                                                                  dguess, h->cnt);
   HIPCHK(h, hipGetLastError());
