@@ -509,11 +509,12 @@ int m2cx_autotune(m2cx_solver* h, int* variant, float* ms_per_variant);
 int m2cx_set_tile(m2cx_solver* h, int variant);
 
 /* No counterpart in the reference (scheduling only).  With material
- * interfaces, each stage runs the stage kernel's tiles that touch no
- * interface face on a second stream while the interface Riemann problems
- * are solved, and the other tiles after them (default: on; results are the
- * same either way).  m2cx_set_overlap(h, 0) runs one launch per stage after
- * the Riemann solve, e.g. to time the stage kernel alone. */
+ * interfaces, each stage runs the tiles whose cells and their surroundings
+ * hold one material, and the level set where it need not wait, on a second
+ * stream while the interface Riemann problems are solved, and the other tiles
+ * after them (default: on; results are the same either way).
+ * m2cx_set_overlap(h, 0) runs them one after another, e.g. to time the stage
+ * kernels alone. */
 int m2cx_set_overlap(m2cx_solver* h, int on);
 
 /* ------------------------------------------------------------------ */
