@@ -554,8 +554,15 @@ __device__ __forceinline__ void ustage_tile(const StageArgs& a, int tile) {
   else ustage_body<MODE, BX, BY, BZ, HLLC, GEN>(a, tile, E, sF);
 }
 
+// Waves per SIMD the compiler keeps the kernel's registers to: three for HLLC and
+// primitive variables (168 registers; the ensemble's form took 169 by itself and
+// ran two: 12 members of 48^3 to 128^3, beside the Riemann launch, 2.42 ms per
+// launch against 1.36 ms), two, as they are, for the eigenvectors of the others
+// (185 to 199).
+constexpr int ustage_waves(bool hllc, bool gen) { return hllc && !gen ? 3 : 2; }
+
 template <int MODE, int BX, int BY, int BZ, bool HLLC, bool GEN>
-__global__ void __launch_bounds__(BX * BY * BZ) k_stage_u(StageArgs a) {
+__global__ void __launch_bounds__(BX * BY * BZ, ustage_waves(HLLC, GEN)) k_stage_u(StageArgs a) {
   // read in place, as in k_stage
   const StageArgs& ar = *(const StageArgs*)__builtin_amdgcn_kernarg_segment_ptr();
   const DevGrid& g = ar.g;
@@ -567,8 +574,8 @@ __global__ void __launch_bounds__(BX * BY * BZ) k_stage_u(StageArgs a) {
 
 // the members of an ensemble in one launch, as k_stage_multi
 template <int MODE, int BX, int BY, int BZ, bool HLLC, bool GEN>
-__global__ void __launch_bounds__(BX * BY * BZ) k_stage_u_multi(const StageArgs* __restrict__ tab,
-                                                                 const int* __restrict__ toff, int nm) {
+__global__ void __launch_bounds__(BX * BY * BZ, ustage_waves(HLLC, GEN))
+    k_stage_u_multi(const StageArgs* __restrict__ tab, const int* __restrict__ toff, int nm) {
   const int total = toff[nm];
   const int t = xcd_tile(total);
   if (t >= total) return;
