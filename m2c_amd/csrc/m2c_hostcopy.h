@@ -7,6 +7,8 @@
 // in order while a few threads copy them to (from) the caller's array.  The
 // ring belongs to one solver and is allocated at its first large copy.
 // The fields of a 256^3 solver (0.75 GB) to fresh host arrays: 85 -> 30 ms.
+// Memory that the link reaches itself (pinned or managed by the caller) is left
+// to the runtime: 256 MB take 4.7 ms directly, 6.7 ms through the ring.
 #pragma once
 #include <hip/hip_runtime.h>
 #include <sched.h>
@@ -77,6 +79,16 @@ class HostPipe {
     return (int)std::min<size_t>(chunks, (size_t)std::max(1, std::min(cpus, MAX_THREADS)));
   }
 
+  // memory the runtime knows nothing of, which the link cannot reach itself
+  static bool pageable(const void* p) {
+    hipPointerAttribute_t a;
+    if (hipPointerGetAttributes(&a, p) != hipSuccess) {  // how older runtimes say so
+      (void)hipGetLastError();
+      return true;
+    }
+    return a.type == hipMemoryTypeUnregistered;
+  }
+
   static hipError_t plain(char* host, char* dev, size_t bytes, hipStream_t st, bool up) {
     hipError_t e = up ? hipMemcpyAsync(dev, host, bytes, hipMemcpyHostToDevice, st)
                       : hipMemcpyAsync(host, dev, bytes, hipMemcpyDeviceToHost, st);
@@ -84,7 +96,8 @@ class HostPipe {
   }
 
   hipError_t run(int device, char* host, char* dev, size_t bytes, hipStream_t st, bool up) {
-    if (bytes < LEAST || !ready()) return plain(host, dev, bytes, st, up);
+    if (bytes < LEAST || !pageable(host) || !pageable(host + bytes - 1) || !ready())
+      return plain(host, dev, bytes, st, up);
     const size_t n = (bytes + CHUNK - 1) / CHUNK;
     // `host_done` counts per ring slot the chunks its threads have finished
     // with; `linked` is the number of chunks given to the link (to_host)

@@ -2,6 +2,7 @@
 the copies change: below and above the threshold of the pinned ring, whole and
 partial last chunks, fewer and more chunks than the ring holds, two solvers
 copying from two threads at once, and a state stepped after an upload."""
+import ctypes as C
 import threading
 
 import numpy as np
@@ -71,3 +72,23 @@ def test_steps_between_large_copies():
     o.set_state(V, ID, None)
     o.run_steps(2)
     assert np.array_equal(gpu.get_state()[0][1:-1, 1:-1, 1:-1], o.get_state()[0][1:-1, 1:-1, 1:-1])
+
+
+@pytest.mark.parametrize("n", [(58, 58, 58), (126, 126, 126)])
+def test_pinned_arrays_of_the_caller(n):
+    """Fields to and from arrays the caller has pinned (through the runtime
+    that the library has loaded, see test_zz_no_alloc.py)."""
+    sol = _solver(n)
+    hip = C.CDLL("libamdhip64.so.7")
+    V, ID, Phi = _fields(sol.shape, 3)
+    same = []
+    for field, a in ((abi.FIELD_V, V), (abi.FIELD_ID, ID), (abi.FIELD_PHI, Phi)):
+        p = C.c_void_p()
+        assert hip.hipHostMalloc(C.byref(p), C.c_size_t(a.nbytes), 0) == 0
+        C.memmove(p, a.ctypes.data, a.nbytes)
+        sol._check(sol.L.m2cx_upload(sol.h, field, p))
+        C.memset(p, 0xFF, a.nbytes)
+        sol._check(sol.L.m2cx_download(sol.h, field, p))
+        same.append(C.string_at(p, a.nbytes) == a.tobytes())
+        assert hip.hipHostFree(p) == 0
+    assert same == [True, True, True]
