@@ -84,7 +84,8 @@ struct m2cx_solver {
   // the others run the one-material kernel when the scheme has one (ustage).
   // A solver of one material without inactive cells has no mixed tile and
   // needs no flags, unless its steps are captured (flags_always: the IDs may
-  // be uploaded anew between replays).
+  // be uploaded anew between replays).  Schemes without that kernel need them
+  // for the overlap alone.
   unsigned char* tflag = nullptr;
   bool ustage = false, has_inactive = false, flags_always = false;
   // level-set reinitialization
@@ -797,8 +798,10 @@ int m2cx_get_time(m2cx_solver* h, double* t, double* dt, int* time_step) {
   return 0;
 }
 
-// whether the stage launches of the next step need the tile flags
-static bool needs_tflags(const m2cx_solver* h) { return h->multimat || h->has_inactive || h->flags_always; }
+// whether the stage launches tell mixed tiles from those of one material
+static bool needs_mixed(const m2cx_solver* h) {
+  return h->ustage && (h->multimat || h->has_inactive || h->flags_always);
+}
 
 static StageArgs stage_args(m2cx_solver* h, int vin, int vout, int mode) {
   StageArgs a{};
@@ -817,7 +820,7 @@ static StageArgs stage_args(m2cx_solver* h, int vin, int vout, int mode) {
   a.mode = mode;
   a.cnt = h->cnt;
   a.gflux = h->gflux;
-  a.tflag = needs_tflags(h) ? h->tflag : nullptr;
+  a.tflag = (!h->ustage || needs_mixed(h)) ? h->tflag : nullptr;
   return a;
 }
 
@@ -904,7 +907,7 @@ static int autotune(m2cx_solver* h, float* ms_out) {
   float best_ms = 1e30f;
   for (int v = 0; v < kNumTiles; v++) {
     h->tile = v;
-    if (needs_tflags(h)) tile_flags(h);
+    if (needs_mixed(h)) tile_flags(h);
     launch_stage(h, 0, -1, MODE_RESIDUAL);  // warm
     HIPCHK(h, hipEventRecord(e0, h->stream));
     for (int r = 0; r < 3; r++) launch_stage(h, 0, -1, MODE_RESIDUAL);
@@ -957,7 +960,7 @@ static void recon_stage(m2cx_solver* h, int vin) {
   if (h->rflag) {
     // where the one-material stage kernel runs, its tiles' cells are marked by
     // code for one material and the others by the general code
-    const bool u = h->ustage, rest = !u || needs_tflags(h);
+    const bool u = h->ustage, rest = !u || needs_mixed(h);
     int tx, ty, tz;
     stage_tile_dims(h, tx, ty, tz);
     if (u) recon_flags_launch_u(stage_args(h, vin, -1, MODE_RESIDUAL), h->rflag, h->stream);
@@ -1030,7 +1033,7 @@ int m2cx_compute_residual(m2cx_solver* h, int v_field, int capture_riemann) {
   HIPCHK(h, hipSetDevice(h->device));
   if (int rc = ensure_slab(h)) return rc;
   if (h->multimat) mp_classify(h->mp, h->g, h->s, h->ID, h->cnt, h->stream);
-  if (needs_tflags(h)) tile_flags(h);
+  if (needs_mixed(h)) tile_flags(h);
   interface_stage(h, v_field, capture_riemann);
   launch_stage(h, v_field, -1, MODE_RESIDUAL);
   HIPCHK(h, hipGetLastError());
@@ -1569,7 +1572,7 @@ static int step_kernels(m2cx_solver* h) {
     swap_ls(h, q);
     if (unbuilt) return fail(h, M2CX_E_ARG, "the narrow band of the level set has not been constructed");
   }
-  if (needs_tflags(h)) tile_flags(h);
+  if (h->overlap || needs_mixed(h)) tile_flags(h);
   if (ti == M2CX_TI_FORWARD_EULER && h->overlap) {
     split_stage(h, StageSpec{0, 1, MODE_FE, 1, 0, -1});
     for (int p = 0; p < 5; p++) std::swap(h->V[0][p], h->V[1][p]);
@@ -2090,8 +2093,8 @@ struct m2cx_ensemble {
   int lanes = 4 * RIEM_LANES, pathcap = 512;
   hipGraph_t graph = nullptr;
   hipGraphExec_t exec = nullptr;
-  // members' stage tiles without interface faces run on stream2 while the
-  // batched Riemann launch runs on stream
+  // members' stage tiles of one material run on stream2 while the batched
+  // Riemann launch runs on stream
   bool overlap = false;
   hipStream_t stream2 = nullptr;
   hipEvent_t ev_fork = nullptr, ev_join = nullptr;
@@ -2162,7 +2165,8 @@ static void ensemble_step(m2cx_ensemble* e) {
   stage_specs(e->ti, sp);
   // split: the member's stage launch is divided by tiles as in split_stage
   auto split = [e](const m2cx_solver* h) { return e->overlap && ens_riemann_member(h); };
-  for (m2cx_solver* h : act) tile_flags(h);
+  for (m2cx_solver* h : act)
+    if (split(h) || needs_mixed(h)) tile_flags(h);
   for (int q = 0; q < e->nstages; q++) {
     for (m2cx_solver* h : act) {
       recon_stage(h, sp[q].vin);
@@ -2177,8 +2181,8 @@ static void ensemble_step(m2cx_ensemble* e) {
       k_riem_count<<<e->nriem, 256, 0, e->stream>>>(e->dmem[q]);
     }
     if (e->overlap) {
-      // the stage tiles of all members: one launch per tile shape, tiles
-      // without interface faces beside the Riemann launch, the others after it
+      // the stage tiles of all members: one launch per class, tiles of one
+      // material beside the Riemann launch, the mixed ones after it
       hipStreamWaitEvent(e->stream2, e->ev_fork, 0);
       for (const auto& c : e->classes) launch_class(c, q, 1, sp[q].mode, e->stream2);
       for (m2cx_solver* h : act)

@@ -1,0 +1,69 @@
+"""Counts the kernels that steps of small solvers launch, by name, and prints
+them as JSON: {case: {kernel: launches}}.  Run as a program of its own: the
+profiler belongs to torch, which has to bring up the runtime before the
+library does."""
+import json
+import os
+import re
+import sys
+
+import torch
+from torch.profiler import ProfilerActivity, profile
+
+sys.path.insert(0, os.path.dirname(os.path.dirname(os.path.abspath(__file__))))
+from m2c_amd import abi, configs, runtime  # noqa: E402
+
+
+def counted(work):
+    with profile(activities=[ProfilerActivity.CPU, ProfilerActivity.CUDA]) as p:
+        work()
+        torch.cuda.synchronize()
+    out = {}
+    for e in p.key_averages():
+        m = re.search(r"m2c::(k_\w+)", e.key)
+        if m:
+            out[m.group(1)] = out.get(m.group(1), 0) + e.count
+    return out
+
+
+def bubble(overlap, **scheme):
+    g, mats, nmat, s, V, ID, Phi = configs.c2_shock_bubble(24, radius=0.27)
+    for k, v in scheme.items():
+        setattr(s, k, v)
+    sol = runtime.Solver(g, mats, nmat, s)
+    sol.set_overlap(overlap)
+    sol.set_state(V, ID, Phi)
+    sol.run_steps(1)
+    return counted(lambda: sol.run_steps(1))
+
+
+def gas(inactive, **scheme):
+    g, mats, nmat, s, V, ID, _ = configs.c1_sod((32, 8, 8))
+    for k, v in scheme.items():
+        setattr(s, k, v)
+    sol = runtime.Solver(g, mats, nmat, s)
+    ID = ID.copy()
+    if inactive:
+        ID[3:5, 3:5, 10:14] = nmat
+    sol.set_state(V, ID)
+    sol.run_steps(1)
+    return counted(lambda: sol.run_steps(1))
+
+
+def main():
+    torch.zeros(1, device="cuda")
+    constant = dict(rec_type=abi.REC_CONSTANT)
+    out = {
+        "bubble": bubble(True),
+        "bubble, one stream": bubble(False),
+        "bubble, constant": bubble(True, **constant),
+        "bubble, constant, one stream": bubble(False, **constant),
+        "gas": gas(False),
+        "gas, inactive cells": gas(True),
+        "gas, inactive cells, constant": gas(True, **constant),
+    }
+    print(json.dumps(out))
+
+
+if __name__ == "__main__":
+    main()

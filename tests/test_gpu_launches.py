@@ -1,0 +1,30 @@
+"""Which kernels a step launches: the marks of the mixed stage tiles are made
+where something reads them."""
+import json
+import os
+import subprocess
+import sys
+
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def launches():
+    r = subprocess.run([sys.executable, os.path.join(os.path.dirname(os.path.abspath(__file__)), "kernel_launches.py")],
+                       capture_output=True, text=True, timeout=100)
+    assert r.returncode == 0, r.stderr[-2000:]
+    return json.loads(r.stdout.split("\n")[-2])
+
+
+@pytest.mark.parametrize("case,marks", [
+    ("bubble", 1), ("bubble, one stream", 1),  # the mixed tiles go to the general kernel
+    # constant reconstruction: no other kernel, marks for the overlap alone
+    ("bubble, constant", 1), ("bubble, constant, one stream", 0),
+    ("gas", 0), ("gas, inactive cells", 1), ("gas, inactive cells, constant", 0),
+])
+def test_marks_of_the_stage_tiles(launches, case, marks):
+    n = launches[case]
+    assert n.get("k_dt") == 1  # one step was seen
+    assert n.get("k_tile_mixed", 0) == marks, n
