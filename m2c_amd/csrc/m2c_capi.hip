@@ -876,9 +876,11 @@ static void tile_flags(m2cx_solver* h) {
 // current state (results are identical across variants: each face flux is
 // computed from the same inputs whichever thread does it, and each cell
 // accumulates its six faces in the same order) and keeps the fastest.  The
-// choice is cached per grid shape and scheme for the process.
-static std::map<std::tuple<int, int, int, int, int, int>, int>& tile_cache() {
-  static std::map<std::tuple<int, int, int, int, int, int>, int> c;
+// choice is cached per grid shape and scheme for the process, apart for the
+// solvers with and without a one-material kernel.
+using TileKey = std::tuple<int, int, int, int, int, int, int>;
+static std::map<TileKey, int>& tile_cache() {
+  static std::map<TileKey, int> c;
   return c;
 }
 
@@ -887,7 +889,7 @@ static int autotune(m2cx_solver* h, float* ms_out) {
     h->tile = 0;
     return 0;
   }
-  const auto key = std::make_tuple(h->g.NX, h->g.NY, h->g.NZ, h->s.flux, h->s.limiter, (int)h->multimat);
+  const TileKey key{h->g.NX, h->g.NY, h->g.NZ, h->s.flux, h->s.limiter, (int)h->multimat, (int)h->ustage};
   auto it = tile_cache().find(key);
   if (it != tile_cache().end() && !ms_out) {
     h->tile = it->second;
@@ -924,7 +926,7 @@ static int autotune(m2cx_solver* h, float* ms_out) {
   HIPCHK(h, hipStreamSynchronize(h->stream));
   HIPCHK(h, hipMemcpy(&h->cnt->error, &err0, sizeof(int), hipMemcpyHostToDevice));
   h->tile = best;
-  tile_cache()[key] = best;
+  if (!h->rflag) tile_cache()[key] = best;  // its four trials were of one shape
   return 0;
 }
 }  // extern "C++"

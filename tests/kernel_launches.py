@@ -50,6 +50,19 @@ def gas(inactive, **scheme):
     return counted(lambda: sol.run_steps(1))
 
 
+def tuned(n, first, second):
+    """The first step of a solver after another of its size tuned its tiles."""
+    sols = []
+    for scheme in (first, second):
+        g, mats, nmat, s, V, ID, _ = configs.c1_sod(n)
+        for k, v in scheme.items():
+            setattr(s, k, v)
+        sols.append(runtime.Solver(g, mats, nmat, s))
+        sols[-1].set_state(V, ID)
+    sols[0].autotune()
+    return counted(lambda: sols[1].run_steps(1))
+
+
 def main():
     torch.zeros(1, device="cuda")
     constant = dict(rec_type=abi.REC_CONSTANT)
@@ -61,6 +74,9 @@ def main():
         "gas": gas(False),
         "gas, inactive cells": gas(True),
         "gas, inactive cells, constant": gas(True, **constant),
+        "tuned by its like": tuned((64, 64, 65), {}, {}),
+        "tuned by constant": tuned((64, 64, 66), constant, {}),
+        "tuned by characteristic": tuned((64, 64, 67), dict(var_type=abi.VAR_CONSERVATIVE_CHARACTERISTIC), {}),
     }
     print(json.dumps(out))
 

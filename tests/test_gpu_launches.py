@@ -1,5 +1,5 @@
 """Which kernels a step launches: the marks of the mixed stage tiles are made
-where something reads them."""
+where something reads them, and tile shapes are tuned per stage kernel."""
 import json
 import os
 import subprocess
@@ -28,3 +28,10 @@ def test_marks_of_the_stage_tiles(launches, case, marks):
     n = launches[case]
     assert n.get("k_dt") == 1  # one step was seen
     assert n.get("k_tile_mixed", 0) == marks, n
+
+
+@pytest.mark.parametrize("case,trials", [("tuned by its like", 0), ("tuned by constant", 16),
+                                         ("tuned by characteristic", 16)])
+def test_tile_shapes_are_tuned_for_the_kernel_that_runs(launches, case, trials):
+    """Four trials of each of the four shapes, then the two stages of a step."""
+    assert launches[case]["k_stage_u"] == trials + 2, launches[case]
