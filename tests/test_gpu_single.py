@@ -231,3 +231,16 @@ def test_autotune_reports_all_variants():
     gpu.set_state(V, ID, Phi)
     v, ms = gpu.autotune()
     assert 0 <= v < 4 and all(m > 0 for m in ms) and ms[v] == min(ms)
+
+
+def test_trials_of_the_tile_shapes_are_not_timed():
+    from m2c_amd import runtime
+    g, mats, nmat, s, V, ID, _ = configs.c1_sod((64, 66, 65))  # a size no other test tunes
+    gpu = runtime.Solver(g, mats, nmat, s)
+    gpu.set_state(V, ID)
+    gpu.profile(True)
+    gpu.run_steps(3)
+    gpu.autotune()
+    assert gpu.kernel_time("stage")[1] == 6
+    gpu.run_steps(1)
+    assert gpu.kernel_time("stage")[1] == 8
