@@ -88,6 +88,7 @@ struct m2cx_solver {
   // for the overlap alone.
   unsigned char* tflag = nullptr;
   bool ustage = false, has_inactive = false, flags_always = false;
+  int id_uploads = 0;
   // level-set reinitialization
   RBuf rb{};
   double reinit_cfl = 0.8;  // the reinitializer's CFL, lowered by its failsafe
@@ -718,12 +719,13 @@ int m2cx_upload(m2cx_solver* h, int field, const void* host) {
   const long n = h->ncells;
   if (field == M2CX_FIELD_ID) {
     HIPCHK(h, h->pipe.to_device(h->device, h->staging_i, host, n * 4, h->stream));
-    k_i32_to_u8<<<grid_blocks(n), 256, 0, h->stream>>>(h->staging_i, h->ID, n, h->s.inactive, &h->cnt->inactive_seen);
+    k_i32_to_u8<<<grid_blocks(n), 256, 0, h->stream>>>(h->staging_i, h->ID, n, h->s.inactive, &h->cnt->inactive_seen,
+                                                        ++h->id_uploads);
     if (!h->multimat) {
       int seen = 0;
       HIPCHK(h, hipMemcpyAsync(&seen, &h->cnt->inactive_seen, sizeof seen, hipMemcpyDeviceToHost, h->stream));
       HIPCHK(h, hipStreamSynchronize(h->stream));
-      h->has_inactive = seen != 0;
+      h->has_inactive = seen == h->id_uploads;
     }
   } else if (field == M2CX_FIELD_PHI) {
     if (!h->mp.phi) return fail(h, M2CX_E_ARG, "no level set");
@@ -2515,7 +2517,7 @@ int m2cx_initialize(m2cx_solver* h, const double* default_state, int default_id,
                                                         h->sch.ls_materialid, diag);
   // boundary fill: state, ghost IDs, level set (ApplyBoundaryConditions,
   // UpdateMaterialIDAtGhostNodes, LevelSetOperator::ApplyBoundaryConditions)
-  if (default_id == h->s.inactive) h->has_inactive = true;
+  h->has_inactive = default_id == h->s.inactive;
   for (const InitGeom& b : G) h->has_inactive = h->has_inactive || b.id == h->s.inactive;
   k_apply_bc<<<grid_blocks(nin), 256, 0, h->stream>>>(h->g, f5(h, h->V[0]));
   const long nf = 2L * ((long)h->g.NY * h->g.NZ + (long)h->g.NX * h->g.NZ + (long)h->g.NX * h->g.NY);

@@ -225,15 +225,16 @@ __global__ void k_soa_to_aos(CF5 src, double* __restrict__ dst, int dof, long n)
   for (long c = blockIdx.x * (long)blockDim.x + threadIdx.x; c < n; c += (long)gridDim.x * blockDim.x)
     for (int p = 0; p < dof; p++) dst[c * dof + p] = src(p, c);
 }
-// `seen` is set once some cell holds the material `inactive`
+// `seen` becomes `upload`, the number of this field, if a cell holds the
+// material `inactive`
 __global__ void k_i32_to_u8(const int* __restrict__ src, unsigned char* __restrict__ dst, long n, int inactive,
-                            int* seen) {
+                            int* seen, int upload) {
   bool any = false;
   for (long c = blockIdx.x * (long)blockDim.x + threadIdx.x; c < n; c += (long)gridDim.x * blockDim.x) {
     dst[c] = (unsigned char)src[c];
     any |= (int)(unsigned char)src[c] == inactive;
   }
-  if (any) *seen = 1;
+  if (any) *seen = upload;
 }
 __global__ void k_u8_to_i32(const unsigned char* __restrict__ src, int* __restrict__ dst, long n) {
   for (long c = blockIdx.x * (long)blockDim.x + threadIdx.x; c < n; c += (long)gridDim.x * blockDim.x)

@@ -24,7 +24,7 @@ struct DevCounters {
   double t, dt, cfl, dts, tmax;
   int time_step, pad2;
   unsigned long long unresolved_total;  // cells left unresolved by the state update, summed
-  int inactive_seen;  // an uploaded ID field held the inactive material
+  int inactive_seen;  // number of the last uploaded ID field that held the inactive material
   int pad3;
 };
 

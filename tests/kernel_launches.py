@@ -50,6 +50,26 @@ def gas(inactive, **scheme):
     return counted(lambda: sol.run_steps(1))
 
 
+def gas_again(way):
+    """A solver of one gas that held inactive cells before."""
+    g, mats, nmat, s, V, ID, _ = configs.c1_sod((32, 8, 8))
+    sol = runtime.Solver(g, mats, nmat, s)
+    state = (1.0, 0.0, 0.0, 0.0, 1.0)
+    solid = abi.geometry("sphere", (0.4, 0.1, 0.1), radius=0.1, materialid=nmat, state=state)
+    if way == "upload":
+        held = ID.copy()
+        held[3:5, 3:5, 10:14] = nmat
+        sol.set_state(V, held)
+    else:
+        sol.initialize(state, 0, [solid])
+    with_cells = counted(lambda: sol.run_steps(1))
+    if way == "upload":
+        sol.set_state(V, ID)
+    else:
+        sol.initialize(state, 0, [])
+    return {"with": with_cells, "without": counted(lambda: sol.run_steps(1))}
+
+
 def tuned(n, first, second):
     """The first step of a solver after another of its size tuned its tiles."""
     sols = []
@@ -74,6 +94,8 @@ def main():
         "gas": gas(False),
         "gas, inactive cells": gas(True),
         "gas, inactive cells, constant": gas(True, **constant),
+        "gas again, upload": gas_again("upload"),
+        "gas again, initialize": gas_again("initialize"),
         "tuned by its like": tuned((64, 64, 65), {}, {}),
         "tuned by constant": tuned((64, 64, 66), constant, {}),
         "tuned by characteristic": tuned((64, 64, 67), dict(var_type=abi.VAR_CONSERVATIVE_CHARACTERISTIC), {}),

@@ -35,3 +35,12 @@ def test_marks_of_the_stage_tiles(launches, case, marks):
 def test_tile_shapes_are_tuned_for_the_kernel_that_runs(launches, case, trials):
     """Four trials of each of the four shapes, then the two stages of a step."""
     assert launches[case]["k_stage_u"] == trials + 2, launches[case]
+
+
+@pytest.mark.parametrize("way", ["upload", "initialize"])
+def test_inactive_cells_that_are_gone_cost_nothing(launches, way):
+    """Marks and the general stage kernel while there are inactive cells, and
+    neither once the solver's material IDs are set anew without any."""
+    n = launches["gas again, " + way]
+    assert n["with"]["k_tile_mixed"] == 1 and n["with"]["k_stage"] == n["with"]["k_stage_u"] == 2, n
+    assert "k_tile_mixed" not in n["without"] and "k_stage" not in n["without"] and n["without"]["k_stage_u"] == 2, n
