@@ -242,11 +242,13 @@ static int mat_slot_acquire(m2cx_solver* h) {
   }
   if (slot < 0) return fail(h, M2CX_E_CAPACITY, "too many distinct material tables on one device");
   if (v[slot].refs == 0) {
-    hipError_t e = hipMemcpyToSymbol(HIP_SYMBOL(c_mats), &h->M, sizeof(DevMats), slot * sizeof(DevMats));
-    if (e == hipSuccess) e = stage_set_materials(slot, h->M);
-    if (e == hipSuccess) e = ustage_set_materials_hllc(slot, h->M);
-    if (e == hipSuccess) e = ustage_set_materials_other(slot, h->M);
-    if (e == hipSuccess) e = ustage_set_materials_gen(slot, h->M);
+    // one copy per translation unit, and one wait for them
+    hipError_t e = hipMemcpyToSymbolAsync(HIP_SYMBOL(c_mats), &h->M, sizeof(DevMats), slot * sizeof(DevMats),
+                                          hipMemcpyHostToDevice, h->stream);
+    for (auto set : {stage_set_materials, ustage_set_materials_hllc, ustage_set_materials_other,
+                     ustage_set_materials_gen})
+      if (e == hipSuccess) e = set(slot, h->M, h->stream);
+    if (e == hipSuccess) e = hipStreamSynchronize(h->stream);
     if (e != hipSuccess) return fail(h, M2CX_E_HIP, std::string("material table upload: ") + hipGetErrorString(e));
     v[slot].m = h->M;
   }

@@ -57,8 +57,9 @@ void stage_launch_multi(const StageArgs* tab, const int* toff, int nm, int ntile
   }
 }
 
-hipError_t stage_set_materials(int slot, const DevMats& m) {
-  return hipMemcpyToSymbol(HIP_SYMBOL(c_mats), &m, sizeof(DevMats), slot * sizeof(DevMats));
+hipError_t stage_set_materials(int slot, const DevMats& m, hipStream_t st) {
+  return hipMemcpyToSymbolAsync(HIP_SYMBOL(c_mats), &m, sizeof(DevMats), slot * sizeof(DevMats), hipMemcpyHostToDevice,
+                                st);
 }
 
 }  // namespace m2c

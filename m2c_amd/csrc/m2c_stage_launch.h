@@ -29,8 +29,8 @@ void stage_launch_gen(const StageArgs& a, int mode, hipStream_t st);
 // the members of an ensemble: argument table and prefix sums of their tiles
 void stage_launch_multi(const StageArgs* tab, const int* toff, int nm, int ntiles, int mode, int variant,
                         hipStream_t st);
-// slot of the material tables in each unit's constant memory
-hipError_t stage_set_materials(int slot, const DevMats& m);
+// slot of the material tables in each unit's constant memory (enqueued on st)
+hipError_t stage_set_materials(int slot, const DevMats& m, hipStream_t st);
 
 // tiles of one material (those that a.tflag, when given, does not mark), for
 // the HLLC flux and for the others
@@ -44,8 +44,8 @@ void ustage_launch_multi_other(const StageArgs* tab, const int* toff, int nm, in
 void ustage_launch_gen(const StageArgs& a, int mode, hipStream_t st);
 // the marks of k_recon_flags on the tiles of one material
 void recon_flags_launch_u(const StageArgs& a, unsigned char* flag, hipStream_t st);
-hipError_t ustage_set_materials_gen(int slot, const DevMats& m);
-hipError_t ustage_set_materials_hllc(int slot, const DevMats& m);
-hipError_t ustage_set_materials_other(int slot, const DevMats& m);
+hipError_t ustage_set_materials_gen(int slot, const DevMats& m, hipStream_t st);
+hipError_t ustage_set_materials_hllc(int slot, const DevMats& m, hipStream_t st);
+hipError_t ustage_set_materials_other(int slot, const DevMats& m, hipStream_t st);
 
 }  // namespace m2c

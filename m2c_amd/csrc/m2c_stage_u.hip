@@ -11,8 +11,9 @@ void ustage_launch_multi_hllc(const StageArgs* tab, const int* toff, int nm, int
                               hipStream_t st) {
   launch_shape_multi<true>(tab, toff, nm, ntiles, mode, variant, st);
 }
-hipError_t ustage_set_materials_hllc(int slot, const DevMats& m) {
-  return hipMemcpyToSymbol(HIP_SYMBOL(c_mats), &m, sizeof(DevMats), slot * sizeof(DevMats));
+hipError_t ustage_set_materials_hllc(int slot, const DevMats& m, hipStream_t st) {
+  return hipMemcpyToSymbolAsync(HIP_SYMBOL(c_mats), &m, sizeof(DevMats), slot * sizeof(DevMats), hipMemcpyHostToDevice,
+                                st);
 }
 
 }  // namespace m2c

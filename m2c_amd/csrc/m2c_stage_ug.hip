@@ -72,8 +72,9 @@ void recon_flags_launch_u(const StageArgs& a, unsigned char* flag, hipStream_t s
   constexpr int X = kTiles[kGenTile].bx, Y = kTiles[kGenTile].by, Z = kTiles[kGenTile].bz;
   k_recon_flags_u<X, Y, Z><<<stage_grid(stage_tiles(a.g, X, Y, Z)), X * Y * Z, 0, st>>>(a, flag);
 }
-hipError_t ustage_set_materials_gen(int slot, const DevMats& m) {
-  return hipMemcpyToSymbol(HIP_SYMBOL(c_mats), &m, sizeof(DevMats), slot * sizeof(DevMats));
+hipError_t ustage_set_materials_gen(int slot, const DevMats& m, hipStream_t st) {
+  return hipMemcpyToSymbolAsync(HIP_SYMBOL(c_mats), &m, sizeof(DevMats), slot * sizeof(DevMats), hipMemcpyHostToDevice,
+                                st);
 }
 
 }  // namespace m2c

@@ -1,5 +1,5 @@
-"""Counts the kernels that steps of small solvers launch, by name, and prints
-them as JSON: {case: {kernel: launches}}.  Run as a program of its own: the
+"""Counts the kernels that steps of small solvers launch and the runtime calls
+they make, by name, and prints them as JSON: {case: {name: calls}}.  Run as a program of its own: the
 profiler belongs to torch, which has to bring up the runtime before the
 library does."""
 import json
@@ -20,7 +20,7 @@ def counted(work):
         torch.cuda.synchronize()
     out = {}
     for e in p.key_averages():
-        m = re.search(r"m2c::(k_\w+)", e.key)
+        m = re.search(r"m2c::(k_\w+)", e.key) or re.match(r"(hip\w+)$", e.key)
         if m:
             out[m.group(1)] = out.get(m.group(1), 0) + e.count
     return out
@@ -48,6 +48,14 @@ def gas(inactive, **scheme):
     sol.set_state(V, ID)
     sol.run_steps(1)
     return counted(lambda: sol.run_steps(1))
+
+
+def new_materials():
+    """A solver with materials that no other has."""
+    g, _, _, s, _, _, _ = configs.c1_sod((16, 8, 8))
+    mats = abi.materials(abi.material("SG", gamma=1.23))
+    made = []
+    return counted(lambda: made.append(runtime.Solver(g, mats, 1, s)))
 
 
 def gas_again(way):
@@ -94,6 +102,7 @@ def main():
         "gas": gas(False),
         "gas, inactive cells": gas(True),
         "gas, inactive cells, constant": gas(True, **constant),
+        "new materials": new_materials(),
         "gas again, upload": gas_again("upload"),
         "gas again, initialize": gas_again("initialize"),
         "tuned by its like": tuned((64, 64, 65), {}, {}),

@@ -44,3 +44,10 @@ def test_inactive_cells_that_are_gone_cost_nothing(launches, way):
     n = launches["gas again, " + way]
     assert n["with"]["k_tile_mixed"] == 1 and n["with"]["k_stage"] == n["with"]["k_stage_u"] == 2, n
     assert "k_tile_mixed" not in n["without"] and "k_stage" not in n["without"] and n["without"]["k_stage_u"] == 2, n
+
+
+def test_material_tables_are_written_together(launches):
+    """A new table goes to each translation unit's copy without a wait in
+    between."""
+    n = launches["new materials"]
+    assert n.get("hipMemcpyToSymbolAsync", 0) > 0 and "hipMemcpyToSymbol" not in n, n
