@@ -31,3 +31,6 @@ mv -f libm2c_amd_facade.so.tmp libm2c_amd_facade.so
 $CXX -O2 -std=c++17 -fPIC -shared -Wall -Wextra -I../include -o ../tests/libfacade_driver.so.tmp \
   ../tests/facade_driver.cpp -L. -lm2c_amd_facade -lm2c_amd -Wl,-rpath,'$ORIGIN/../m2c_amd'
 mv -f ../tests/libfacade_driver.so.tmp ../tests/libfacade_driver.so
+# the quotients and roots of m2c_exactdiv.h over arrays, for their test
+$HIPCC $FLAGS -shared -o ../tests/libexactdiv.so.tmp ../tests/exactdiv_driver.hip
+mv -f ../tests/libexactdiv.so.tmp ../tests/libexactdiv.so
