@@ -191,3 +191,56 @@ def test_ensemble_at_the_c4_member_sizes():
     assert rc == sum(a[3] for a in alone)
     _same_as_alone(alone, members)
     ens.close()
+
+
+def test_ensemble_of_every_stage_kernel():
+    """Members on each form of the stage: the one-material kernel for HLLC, for
+    Roe and for LLF (one launch for both), on two tile shapes, the one for
+    other reconstruction variables, and the general kernel alone (constant
+    reconstruction), on grids with tiles of one material and mixed ones."""
+    from m2c_amd import runtime
+    cases = configs.c4_instances(count=8, seed=21, edges=(33, 36, 40))
+    schemes = [dict(), dict(flux=abi.FLUX_ROE), dict(flux=abi.FLUX_LLF, limiter=abi.LIM_GMM), dict(limiter=abi.LIM_GMM),
+               dict(flux=abi.FLUX_ROE, var_type=abi.VAR_CONSERVATIVE_CHARACTERISTIC, limiter=abi.LIM_GMM),
+               dict(var_type=abi.VAR_PRIMITIVE_CHARACTERISTIC), dict(rec_type=abi.REC_CONSTANT),
+               dict(flux=abi.FLUX_ROE, riemann_normal=abi.RNORMAL_AVERAGE)]
+
+    def prep(i, s):
+        for k, v in schemes[i].items():
+            setattr(s, k, v)
+
+    alone, members = _alone_and_members(cases, 4, prep)
+    for q in (1, 3):
+        members[q].set_tile(2)
+    ens = runtime.Ensemble(members)
+    ens.run_steps(1)
+    ens.run_steps(3)
+    _same_as_alone(alone, members)
+    ens.close()
+
+
+@pytest.mark.parametrize("var", [abi.VAR_PRIMITIVE, abi.VAR_CONSERVATIVE_CHARACTERISTIC])
+def test_one_material_member_given_inactive_cells_between_replays(var):
+    """The captured step marks its tiles anew: material IDs uploaded between two
+    calls, with inactive cells and without, take effect as they do alone."""
+    from m2c_amd import runtime
+    g, mats, nmat, s, V, ID, _ = configs.c1_sod((40, 18, 13))
+    s.integrator, s.var_type = abi.TI_RK3, var
+    held = ID.copy()
+    held[5:8, 7:9, 20:23] = nmat
+    held[:, 3, 3] = nmat
+    (_, (g2, mats2, nmat2, s2, V2, ID2, Phi2)), = configs.c4_instances(count=1, seed=3, edges=(20,))
+    alone, member, other = runtime.Solver(g, mats, nmat, s), runtime.Solver(g, mats, nmat, s), \
+        runtime.Solver(g2, mats2, nmat2, s2)
+    member.set_state(V, ID)
+    other.set_state(V2, ID2, Phi2)
+    ens = runtime.Ensemble([member, other])
+    for ids in (ID, held, ID):
+        for sol in (alone, member):
+            sol.set_state(V, ids)  # a step leaves no state of use in inactive cells
+        alone.run_steps(2)
+        ens.run_steps(2)
+        live = ids[1:-1, 1:-1, 1:-1] == 0
+        a, b = (sol.get_state()[0][1:-1, 1:-1, 1:-1][live] for sol in (alone, member))
+        assert np.array_equal(a, b)
+    ens.close()
