@@ -69,6 +69,17 @@ def test_states_outside_the_fast_range(scale):
     _check(mats, prob, riem_min_pressure=-1e-8 * scale, riem_pressure_at_failure=1e-8 * scale)
 
 
+@pytest.mark.parametrize("pair", ["sg-air", "nasg-air"])
+@pytest.mark.parametrize("scale", [1e-60, 1e-30, 1e30, 1e60])
+def test_liquid_states_outside_the_fast_range(pair, scale):
+    """Gas pressures and densities far from the liquid's constants, the liquid
+    itself near its density (NASG has a largest one)."""
+    mats, (dirs, Vm, idm, Vp, idp) = _problems(pair, 200, 3, 0.7)
+    Vp[:, 0] *= scale
+    Vp[:, 4] *= scale
+    _check(mats, (dirs, Vm, idm, Vp, idp), riem_min_pressure=-1e-8 * scale, riem_pressure_at_failure=1e-8 * scale)
+
+
 def test_solves_that_end_in_the_second_pass():
     """Two iterations are too few: every problem is solved again without step
     control."""

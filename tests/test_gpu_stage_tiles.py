@@ -182,6 +182,53 @@ def test_ends_of_the_fast_range(case):
     _same_residual(gpu, o)
 
 
+# exponent ranges of density, velocities and pressure at the ends of the fast
+# arithmetic, as factors on the state
+RANGES = {"denormal": (0, (-323, -280), 0), "tiny": (0, (-300, -100), (-200, 0)), "huge": (60, 15, 90),
+          "vacuum": ((-40, 0), 0, (-40, 0)), "thin": ((-40, 0), (-40, 0), 0), "hot": (0, 0, (0, 70))}
+
+
+# NASG and MG have a largest density
+@pytest.mark.parametrize("case,mat", [(c, m) for c in RANGES for m in MATS if c != "huge" or m in ("sg", "stiff")])
+@pytest.mark.parametrize("flux,limiter,var", [
+    (abi.FLUX_HLLC, abi.LIM_VANALBADA, abi.VAR_PRIMITIVE), (abi.FLUX_HLLC, abi.LIM_GMM, abi.VAR_PRIMITIVE),
+    (abi.FLUX_ROE, abi.LIM_VANALBADA, abi.VAR_PRIMITIVE), (abi.FLUX_HLLC, abi.LIM_VANALBADA, abi.VAR_CONSERVATIVE),
+    (abi.FLUX_HLLC, abi.LIM_VANALBADA, abi.VAR_PRIMITIVE_CHARACTERISTIC),
+    (abi.FLUX_ROE, abi.LIM_GMM, abi.VAR_CONSERVATIVE_CHARACTERISTIC)])
+def test_ends_of_the_fast_range_in_every_form(case, mat, flux, limiter, var):
+    n = (24, 10, 8)
+    rng = np.random.default_rng(11)
+    V = _state(n, 4, False)
+    for q, (r, c) in enumerate(zip(RANGES[case], (slice(0, 1), slice(1, 4), slice(4, 5)))):
+        shape = V[..., c].shape
+        if isinstance(r, tuple):
+            V[..., c] = rng.uniform(0.1, 1.0, shape) * 10.0 ** rng.uniform(r[0], r[1], shape) * (1 if q != 1 else
+                                                                                                 rng.choice([-1, 1], shape))
+        elif r:
+            V[..., c] *= 10.0 ** r
+    gpu, o = _pair(n, MATS[mat], V, flux=flux, limiter=limiter, var_type=var)
+    _same_residual(gpu, o)
+
+
+@pytest.mark.parametrize("comp", [0, 1, 3, 4])
+@pytest.mark.parametrize("mat", ["sg", "nasg"])
+@pytest.mark.parametrize("value,flux,var", [
+    (x, f, q) for f, q, xs in ((abi.FLUX_HLLC, abi.VAR_PRIMITIVE, (np.inf, -np.inf, np.nan)),
+                               (abi.FLUX_HLLC, abi.VAR_CONSERVATIVE_CHARACTERISTIC, (np.inf, -np.inf, np.nan)),
+                               (abi.FLUX_ROE, abi.VAR_PRIMITIVE, (np.nan,)), (abi.FLUX_LLF, abi.VAR_PRIMITIVE, (np.nan,)))
+    for x in xs])
+def test_infinities_and_nan(value, comp, mat, flux, var):
+    """One such value in a cell: the same residual or the same abort.  (Roe and
+    LLF in primitive variables with NaN alone: the reference aborts on an
+    infinite density or pressure that clipping would replace, where these
+    fluxes here go on.)"""
+    n = (24, 10, 8)
+    V = _state(n, 4, False)
+    V[4, 5, 9, comp] = value
+    gpu, o = _pair(n, MATS[mat], V, flux=flux, var_type=var)
+    _same_residual(gpu, o)
+
+
 @pytest.mark.parametrize("water", ["sg", "nasg"])
 @pytest.mark.parametrize("variant", [0, 1, 2, 3])
 def test_mixed_and_one_material_tiles(water, variant):
