@@ -641,7 +641,8 @@ static int create_impl(const m2cx_grid* grid, const m2cx_material* mats, int nma
   for (const TileVariant& t : kTiles)
     mt = std::max(mt, stage_tiles(g, t.bx, t.by, t.bz));
   HIPCHK(h, hipMalloc(&h->tflag, mt));
-  // the one-material stage kernel: what its code leaves out (m2c_stage_u.h)
+  // the one-material stage kernel: what its code leaves out (m2c_stage_u.h); the
+  // coefficients of the meshes built above are 1 wherever the box has an extent
   h->ustage = s.flux != M2CX_FLUX_GODUNOV && s.rec_type == M2CX_REC_LINEAR;
   for (size_t q = 0; q < Acoef.size(); q++)
     h->ustage = h->ustage && Acoef[q] == 1.0 && Bcoef[q] == 1.0 && (s.limiter != M2CX_LIM_VANALBADA || Kcoef[q] == 2);
@@ -1528,7 +1529,10 @@ static int end_of_step(m2cx_solver* h) {
 
 // Cells from which the last stage's level set, which waits for the Riemann
 // launch, runs on stream2: below, that wait costs more than the two launches it
-// hides (a 200-cell tube lost 2.9 % to the event alone; 512x256x256 gains 1.6 %).
+// hides.  Ten RK3 steps after it / beside it, best of twelve: 200-cell tube 2.9 %
+// lost to the event alone; 64^3 62.6 / 63.3 ms; 102^3 73.5 / 71.0; 128^3 128.8 /
+// 128.2, in a narrow band 319 / 314; 160^3 132.8 / 130.7; 203^3 165.9 / 165.7;
+// 256^3 200.9 / 203.5 (each side varies by 2); 512x256x256 590 / 585.
 constexpr long LS_BESIDE_CELLS = 1L << 20;
 
 // One stage with the tiles of one material running on stream2 while the
@@ -2113,9 +2117,9 @@ struct m2cx_ensemble {
   bool overlap = false;
   hipStream_t stream2 = nullptr;
   hipEvent_t ev_fork = nullptr, ev_join = nullptr;
-  // the stage kernel of all split members that share a tile shape, one
-  // launch per stage and phase (k_stage_multi): member tables [stage][phase]
-  // and tile-count prefix sums
+  // the stage of all split members that share a tile shape and a kernel, one
+  // launch per stage and phase (k_stage_u_multi, k_stage_multi): member tables
+  // [stage][phase] and tile-count prefix sums
   struct StageClass {
     int v = 0;                 // tile variant (kTiles index)
     bool ustage = false;       // one-material tiles run k_stage_u_multi
@@ -2275,7 +2279,7 @@ static int ensemble_build(m2cx_ensemble* e) {
       EHIPCHK(e, hipMemcpy(e->dmem[q], tab[q].data(), tab[q].size() * sizeof(RiemMember), hipMemcpyHostToDevice));
   }
   // stage classes: active members of the batched Riemann launch whose stage
-  // kernel is the primitive-variable one, grouped by tile shape
+  // kernel is a primitive-variable one, grouped by tile shape and kernel
   free_classes(e);
   e->classed.clear();
   if (e->overlap) {

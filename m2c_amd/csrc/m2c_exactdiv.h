@@ -4,14 +4,19 @@
 //
 // Method: the hardware's reciprocal (square root) estimate is refined by
 // Newton steps in fused arithmetic, and the quotient (root) corrected by its
-// exactly computed remainder, which gives the correctly rounded result
-// (Markstein, "Computation of elementary functions on the IBM RISC
-// System/6000 processor", IBM J. Res. Dev. 34, 1990).  The remainder is exact,
-// and no intermediate leaves the normal range, for
+// exactly computed remainder (Markstein, "Computation of elementary functions on
+// the IBM RISC System/6000 processor", IBM J. Res. Dev. 34, 1990).  The remainder
+// is exact, and no intermediate leaves the normal range, for
 //   |b| in [2^-900, 2^900], |a| zero or in [2^-900, 2^1000], |a/b| in [2^-1000, 2^1000]
 // for the quotient a/b, and x in [2^-700, 2^900] for the root: callers check
-// their operands and fall back to `/` and sqrt().  (Of a zero numerator the
-// quotient is a zero, whose sign may differ from a/b's.)
+// their operands and fall back to `/` and sqrt().  Markstein's theorem gives the
+// correctly rounded quotient from a correctly rounded reciprocal.  The refined
+// one is that but for denominators whose reciprocal lies within ~2^-100 of the
+// middle of two doubles; that the quotients are the IEEE ones there as well, and
+// the roots, rests on a test: random operands, such denominators, and quotients
+// and roots nearest to the middle of two doubles, all bit for bit.  Of a zero
+// numerator the quotient is a zero, whose sign may differ from a/b's; callers'
+// results are then equal as numbers.
 #pragma once
 #include <hip/hip_runtime.h>
 

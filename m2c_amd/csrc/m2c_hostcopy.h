@@ -1,11 +1,15 @@
 // Copies between device memory and the caller's (pageable) host arrays.
 //
 // A pageable copy of the runtime moves through one staging buffer on one
-// thread, which also takes the page faults of a fresh destination: 8 to 16
-// GB/s on a link that carries 54 GB/s to pinned memory.  Large copies here go
+// thread, which also takes the page faults of a fresh destination: 256 MB take 63
+// ms to a fresh array, 15 ms to one touched before and 9 ms from one, on a link
+// that needs 4.7 ms to or from pinned memory.  Large copies here go
 // through a ring of pinned chunks instead: the link fills (drains) the chunks
-// in order while a few threads copy them to (from) the caller's array.  The
-// ring belongs to one solver and is allocated at its first large copy.
+// in order while a few threads copy them to (from) the caller's array (11, 6.8
+// and 6.6 ms).  The ring, 16 MB of pinned memory, belongs to one solver and is
+// allocated at its first large copy; threads that wait give their time slice
+// away but do not sleep, so that a process held to few CPUs by other means than
+// its affinity mask (which sets their number) pays for the waiting.
 // The fields of a 256^3 solver (0.75 GB) to fresh host arrays: 85 -> 30 ms.
 // Memory that the link reaches itself (pinned or managed by the caller) is left
 // to the runtime: 256 MB take 4.7 ms directly, 6.7 ms through the ring.
@@ -27,8 +31,9 @@ class HostPipe {
   static constexpr size_t CHUNK = 2u << 20;
   static constexpr int RING = 8;
   static constexpr int MAX_THREADS = 8;
-  // smaller copies are left to the runtime: the threads cost about 0.2 ms to
-  // start, and below this the copy takes less than twice that
+  // Smaller copies are left to the runtime.  Measured at 8 MB, ring and runtime:
+  // to a fresh array 0.8 and 1.9 ms, to one touched before 0.33 and 0.51, from
+  // one 0.30 and 0.30; at 6 MB from one 0.24 and 0.23.
   static constexpr size_t LEAST = 8u << 20;
 
   HostPipe() = default;

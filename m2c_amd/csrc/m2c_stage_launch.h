@@ -1,7 +1,7 @@
 // Launches of the fused stage kernels, which have translation units of their
 // own (m2c_stage.hip: the general kernel; m2c_stage_u.hip, m2c_stage_ur.hip,
-// m2c_stage_ug.hip: tiles of one material), so that they build beside the rest of the library.  `variant`:
-// tile shape, an index of kTiles.
+// m2c_stage_ug.hip: tiles of one material), so that they build beside the rest
+// of the library.  `variant`: tile shape, an index of kTiles.
 #pragma once
 #include "m2c_stage.h"
 

@@ -9,8 +9,8 @@
 
 namespace m2c {
 
-// Limited slopes of a cell from the one-sided differences d0, d1 along an axis, with the coefficients of a uniform mesh, A = B = 1 and (van Albada)
-// K = 2: lim_gmm and lim_va with the multiplications by one left out.
+// Limited slopes of a cell from the one-sided differences d0, d1 along an axis,
+// with the coefficients of a uniform mesh, A = B = 1 and (van Albada) K = 2: lim_gmm and lim_va with the multiplications by one left out.
 // The divisions of the five components are formed side by side, and not at
 // all where no lane of the wave has a slope to limit.
 __device__ __forceinline__ void limited(const Scheme& s, const double* d0, const double* d1, double* h) {
@@ -300,9 +300,9 @@ __device__ __forceinline__ void flux_hllc_axis(const DevEos& E, bool z, const do
 }
 
 // Roe and LLF keep the x, y, z order (their sums run over it).  HLLC: compiled
-// for that flux alone; the Roe flux's eigenvectors take 203 registers, two
-// waves per SIMD instead of three (256^3 water: 2.42 ms per launch against
-// 1.86 ms).
+// for that flux alone; with the Roe flux's eigenvectors the kernel takes 197 to
+// 199 registers, two waves per SIMD, without them 167, three (256^3 water: 2.42
+// ms per launch against 1.86 ms).
 template <bool HLLC>
 __device__ __forceinline__ void flux_axis(const DevEos& E, const Scheme& s, int D, const double* Wm, const double* Wp,
                                           double* F, int& err) {

@@ -200,8 +200,8 @@ class Solver:
         return out
 
     def set_overlap(self, on):
-        """Stage kernel tiles without interface faces during the Riemann
-        solve (on, the default) or one launch per stage after it."""
+        """Stage tiles of one material during the Riemann solve and the mixed
+        ones after it (on, the default), or all of them after it."""
         return self._check(self.L.m2cx_set_overlap(self.h, int(bool(on))))
 
     def reinitialize(self, special_maxits=0):
