@@ -220,10 +220,15 @@ static void fill_iface_ls(m2cx_solver* h) {
 
 // Slots of c_mats per device: solvers with byte-identical material tables
 // share one; a slot is rewritten only when it is free (no live solver uses it).
+// A translation unit's copy is written when the first solver that runs its
+// kernels needs it (mat_units): writing it loads the unit's code, and a
+// process's first solver took 13 ms longer with all of them (35 -> 48 ms).
 struct MatSlot {
   DevMats m;
   int refs = 0;
+  unsigned units = 0;  // the copies that hold m
 };
+enum MatUnit : unsigned { UNIT_MAIN = 1, UNIT_STAGE = 2, UNIT_U_HLLC = 4, UNIT_U_OTHER = 8, UNIT_U_GEN = 16 };
 static std::mutex g_slot_mu;
 static std::map<int, std::vector<MatSlot>> g_slots;
 
@@ -242,18 +247,37 @@ static int mat_slot_acquire(m2cx_solver* h) {
   }
   if (slot < 0) return fail(h, M2CX_E_CAPACITY, "too many distinct material tables on one device");
   if (v[slot].refs == 0) {
-    // one copy per translation unit, and one wait for them
-    hipError_t e = hipMemcpyToSymbolAsync(HIP_SYMBOL(c_mats), &h->M, sizeof(DevMats), slot * sizeof(DevMats),
-                                          hipMemcpyHostToDevice, h->stream);
-    for (auto set : {stage_set_materials, ustage_set_materials_hllc, ustage_set_materials_other,
-                     ustage_set_materials_gen})
-      if (e == hipSuccess) e = set(slot, h->M, h->stream);
-    if (e == hipSuccess) e = hipStreamSynchronize(h->stream);
-    if (e != hipSuccess) return fail(h, M2CX_E_HIP, std::string("material table upload: ") + hipGetErrorString(e));
     v[slot].m = h->M;
+    v[slot].units = 0;
   }
   v[slot].refs++;
   h->mset = slot;
+  return 0;
+}
+
+static hipError_t main_set_materials(int slot, const DevMats& m, hipStream_t st) {
+  return hipMemcpyToSymbolAsync(HIP_SYMBOL(c_mats), &m, sizeof(DevMats), slot * sizeof(DevMats), hipMemcpyHostToDevice,
+                                st);
+}
+
+// the solver's table in the copies of `need`: one wait for those not yet written
+static int mat_units(m2cx_solver* h, unsigned need) {
+  std::lock_guard<std::mutex> lk(g_slot_mu);
+  MatSlot& s = g_slots[h->device][h->mset];
+  const unsigned missing = need & ~s.units;
+  if (!missing) return 0;
+  hipError_t e = hipSuccess;
+  auto put = [&](unsigned unit, hipError_t (*set)(int, const DevMats&, hipStream_t)) {
+    if ((missing & unit) && e == hipSuccess) e = set(h->mset, h->M, h->stream);
+  };
+  put(UNIT_MAIN, main_set_materials);
+  put(UNIT_STAGE, stage_set_materials);
+  put(UNIT_U_HLLC, ustage_set_materials_hllc);
+  put(UNIT_U_OTHER, ustage_set_materials_other);
+  put(UNIT_U_GEN, ustage_set_materials_gen);
+  if (e == hipSuccess) e = hipStreamSynchronize(h->stream);
+  if (e != hipSuccess) return fail(h, M2CX_E_HIP, std::string("material table upload: ") + hipGetErrorString(e));
+  s.units |= missing;
   return 0;
 }
 
@@ -647,6 +671,13 @@ static int create_impl(const m2cx_grid* grid, const m2cx_material* mats, int nma
   for (size_t q = 0; q < Acoef.size(); q++)
     h->ustage = h->ustage && Acoef[q] == 1.0 && Bcoef[q] == 1.0 && (s.limiter != M2CX_LIM_VANALBADA || Kcoef[q] == 2);
   for (int q = 0; q < nmat; q++) h->ustage = h->ustage && eos_in_range(M.m[q]);
+  // the general stage kernel besides: where there may be mixed tiles, or (later)
+  // once there are inactive cells or the steps are captured
+  const unsigned own = s.var_type != M2CX_VAR_PRIMITIVE ? UNIT_U_GEN
+                       : s.flux == M2CX_FLUX_HLLC       ? UNIT_U_HLLC
+                                                        : UNIT_U_OTHER;
+  const unsigned general = !h->ustage || h->multimat ? UNIT_STAGE : 0u;
+  if (int rc = mat_units(h, UNIT_MAIN | general | (h->ustage ? own : 0u))) return rc;
   if (h->multimat) fill_iface_ls(h);
   HIPCHK(h, hipStreamSynchronize(h->stream));
   return 0;
@@ -729,6 +760,8 @@ int m2cx_upload(m2cx_solver* h, int field, const void* host) {
       HIPCHK(h, hipMemcpyAsync(&seen, &h->cnt->inactive_seen, sizeof seen, hipMemcpyDeviceToHost, h->stream));
       HIPCHK(h, hipStreamSynchronize(h->stream));
       h->has_inactive = seen == h->id_uploads;
+      if (h->has_inactive)
+        if (int rc = mat_units(h, UNIT_STAGE)) return rc;
     }
   } else if (field == M2CX_FIELD_PHI) {
     if (!h->mp.phi) return fail(h, M2CX_E_ARG, "no level set");
@@ -2374,6 +2407,7 @@ int m2cx_ensemble_create(m2cx_solver* const* members, int n, m2cx_ensemble** out
     h->profile = false;
     h->stream_saved = h->stream;
     if (int rc = ensure_slab(h)) return efail(e, rc, h->err);
+    if (int rc = mat_units(h, UNIT_STAGE)) return efail(e, rc, h->err);  // flags_always
     if (ens_riemann_member(h)) e->nriem++;
   }
   if (const char* env = getenv("M2C_ENSEMBLE_RIEMANN_LANES")) {  // launch-shape override: a multiple of 64
@@ -2525,6 +2559,8 @@ int m2cx_initialize(m2cx_solver* h, const double* default_state, int default_id,
   // UpdateMaterialIDAtGhostNodes, LevelSetOperator::ApplyBoundaryConditions)
   h->has_inactive = default_id == h->s.inactive;
   for (const InitGeom& b : G) h->has_inactive = h->has_inactive || b.id == h->s.inactive;
+  if (h->has_inactive)
+    if (int rc = mat_units(h, UNIT_STAGE)) return rc;
   k_apply_bc<<<grid_blocks(nin), 256, 0, h->stream>>>(h->g, f5(h, h->V[0]));
   const long nf = 2L * ((long)h->g.NY * h->g.NZ + (long)h->g.NX * h->g.NZ + (long)h->g.NX * h->g.NY);
   k_ghost_ids<<<grid_blocks(nf), 256, 0, h->stream>>>(h->g, h->ID);

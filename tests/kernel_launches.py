@@ -51,11 +51,13 @@ def gas(inactive, **scheme):
 
 
 def new_materials():
-    """A solver with materials that no other has."""
+    """A solver with materials that no other has, then one of another flux."""
     g, _, _, s, _, _, _ = configs.c1_sod((16, 8, 8))
     mats = abi.materials(abi.material("SG", gamma=1.23))
     made = []
-    return counted(lambda: made.append(runtime.Solver(g, mats, 1, s)))
+    first = counted(lambda: made.append(runtime.Solver(g, mats, 1, s)))
+    s.flux = abi.FLUX_ROE
+    return first, counted(lambda: made.append(runtime.Solver(g, mats, 1, s)))
 
 
 def gas_again(way):
@@ -94,6 +96,7 @@ def tuned(n, first, second):
 def main():
     torch.zeros(1, device="cuda")
     constant = dict(rec_type=abi.REC_CONSTANT)
+    first, second = new_materials()
     out = {
         "bubble": bubble(True),
         "bubble, one stream": bubble(False),
@@ -102,7 +105,8 @@ def main():
         "gas": gas(False),
         "gas, inactive cells": gas(True),
         "gas, inactive cells, constant": gas(True, **constant),
-        "new materials": new_materials(),
+        "new materials": first,
+        "new materials, roe as well": second,
         "gas again, upload": gas_again("upload"),
         "gas again, initialize": gas_again("initialize"),
         "tuned by its like": tuned((64, 64, 65), {}, {}),

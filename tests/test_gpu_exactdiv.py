@@ -46,8 +46,9 @@ def _same(x, y):
 def test_random_quotients(device, seed):
     rng = np.random.default_rng(seed)
     b = _numbers(rng, N, -900, 900)
-    a = _numbers(rng, N, -900, 1000) if seed % 2 else np.ldexp(b, rng.integers(-900, 900, N)) * rng.uniform(0.5, 2.0, N)
     with np.errstate(over="ignore", under="ignore"):
+        a = (_numbers(rng, N, -900, 1000) if seed % 2 else
+             np.ldexp(b, rng.integers(-900, 900, N)) * rng.uniform(0.5, 2.0, N))
         q = a / b
     keep = (np.abs(a) >= 2.0**-900) & (np.abs(a) <= 2.0**1000) & (np.abs(q) >= 2.0**-1000) & (np.abs(q) <= 2.0**1000)
     assert keep.sum() > N // 4

@@ -46,8 +46,9 @@ def test_inactive_cells_that_are_gone_cost_nothing(launches, way):
     assert "k_tile_mixed" not in n["without"] and "k_stage" not in n["without"] and n["without"]["k_stage_u"] == 2, n
 
 
-def test_material_tables_are_written_together(launches):
-    """A new table goes to each translation unit's copy without a wait in
-    between."""
-    n = launches["new materials"]
-    assert n.get("hipMemcpyToSymbolAsync", 0) > 0 and "hipMemcpyToSymbol" not in n, n
+@pytest.mark.parametrize("case,copies", [("new materials", 2), ("new materials, roe as well", 1)])
+def test_material_tables_are_written_where_they_are_read(launches, case, copies):
+    """A new table goes to the translation units whose kernels its solver runs
+    (each loads its code at the first write), without a wait in between."""
+    n = launches[case]
+    assert n.get("hipMemcpyToSymbolAsync", 0) == copies and "hipMemcpyToSymbol" not in n, n

@@ -140,6 +140,28 @@ def test_inactive_cells_in_a_one_material_solver():
         assert np.array_equal(_g[live], _o[live]), v
 
 
+def test_solvers_of_one_table_on_every_kernel():
+    """Solvers of the same materials, which no other test has, one after another
+    on each form of the stage, all alive: each form finds the table."""
+    n = (20, 12, 9)
+    V = _state(n, 12, False)
+    mat = abi.material("SG", gamma=1.37, pc=0.25)
+    forms = [dict(), dict(flux=abi.FLUX_ROE), dict(var_type=abi.VAR_CONSERVATIVE_CHARACTERISTIC),
+             dict(rec_type=abi.REC_CONSTANT), dict(flux=abi.FLUX_GODUNOV)]
+    pairs = []
+    for kw in forms:
+        pairs.append(_pair(n, mat, V, **kw))
+        for gpu, o in pairs:
+            _same_residual(gpu, o)
+    ID = np.zeros(V.shape[:3], dtype=np.int32)
+    ID[3:5, 4:6, 8:11] = 1
+    for gpu, o in pairs:
+        gpu.upload(abi.FIELD_ID, ID)
+        o.set_state(V, ID, None)
+        live = _inner(ID) == 0
+        assert np.array_equal(_inner(gpu.compute_residual())[live], _inner(o.residual())[live])
+
+
 @pytest.mark.parametrize("var", VARS)
 def test_inactive_cells_in_other_variables(var):
     n = (40, 18, 13)
