@@ -555,10 +555,8 @@ __device__ __forceinline__ void ustage_tile(const StageArgs& a, int tile) {
 }
 
 // Waves per SIMD the compiler keeps the kernel's registers to: three for HLLC and
-// primitive variables (168 registers; the ensemble's form took 169 by itself and
-// ran two: 12 members of 48^3 to 128^3, beside the Riemann launch, 2.42 ms per
-// launch against 1.36 ms), two, as they are, for the eigenvectors of the others
-// (185 to 199).
+// primitive variables (168 registers at most), two, as they are, for the
+// eigenvectors of the others (185 to 199).
 constexpr int ustage_waves(bool hllc, bool gen) { return hllc && !gen ? 3 : 2; }
 
 template <int MODE, int BX, int BY, int BZ, bool HLLC, bool GEN>
@@ -572,9 +570,15 @@ __global__ void __launch_bounds__(BX * BY * BZ, ustage_waves(HLLC, GEN)) k_stage
   ustage_tile<MODE, BX, BY, BZ, HLLC, GEN>(ar, tile);
 }
 
-// the members of an ensemble in one launch, as k_stage_multi
+// The members of an ensemble in one launch, as k_stage_multi.  Two waves per SIMD,
+// also where three would fit: the launch runs beside the batched Riemann launch,
+// four waves per SIMD of 320 registers of which one is resident, and stage waves
+// that take the room a finished one leaves hold the next one back.  At three the
+// stage launches of 12 members of 48^3 to 128^3 were shorter (2.42 -> 1.36 ms) and
+// their steps were not (271 / 268 ms, within the spread); 64 members of 64^3 to
+// 192^3 took 259 to 291 ms per step, by tile shape, instead of 245.
 template <int MODE, int BX, int BY, int BZ, bool HLLC, bool GEN>
-__global__ void __launch_bounds__(BX * BY * BZ, ustage_waves(HLLC, GEN))
+__global__ void __launch_bounds__(BX * BY * BZ) __attribute__((amdgpu_waves_per_eu(2, 2)))
     k_stage_u_multi(const StageArgs* __restrict__ tab, const int* __restrict__ toff, int nm) {
   const int total = toff[nm];
   const int t = xcd_tile(total);
