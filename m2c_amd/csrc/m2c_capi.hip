@@ -512,6 +512,7 @@ static int create_impl(const m2cx_grid* grid, const m2cx_material* mats, int nma
   h->mats.assign(mats, mats + nmat);
   h->device = device;
   HIPCHK(h, hipSetDevice(device));
+  h->pipe.attach(device);
   HIPCHK(h, hipStreamCreateWithFlags(&h->stream, hipStreamNonBlocking));
   if (int rc = scratch_setup(h)) return rc;
   const int NX = grid->nx, NY = grid->ny, NZ = grid->nz;
@@ -732,7 +733,7 @@ int m2cx_upload_levelset(m2cx_solver* h, int ls, const double* host) {
   if (ls < 0 || ls >= h->nls) return fail(h, M2CX_E_ARG, "no such level set");
   HIPCHK(h, hipSetDevice(h->device));
   double* dst = ls == 0 ? h->mp.phi : h->lsx[ls - 1].phi;
-  HIPCHK(h, h->pipe.to_device(h->device, dst, host, h->ncells * 8, h->stream));
+  HIPCHK(h, h->pipe.to_device(dst, host, h->ncells * 8, h->stream));
   return 0;
 }
 
@@ -743,7 +744,7 @@ int m2cx_download_levelset(m2cx_solver* h, int ls, int what, double* host) {
   const bool own = ls == 0;
   const double* src = what == M2CX_LS_PHI ? (own ? h->mp.phi : h->lsx[ls - 1].phi)
                                           : (own ? h->mp.rls : h->lsx[ls - 1].rls);
-  HIPCHK(h, h->pipe.to_host(h->device, host, src, h->ncells * 8, h->stream));
+  HIPCHK(h, h->pipe.to_host(host, src, h->ncells * 8, h->stream));
   return 0;
 }
 
@@ -752,7 +753,7 @@ int m2cx_upload(m2cx_solver* h, int field, const void* host) {
   HIPCHK(h, hipSetDevice(h->device));
   const long n = h->ncells;
   if (field == M2CX_FIELD_ID) {
-    HIPCHK(h, h->pipe.to_device(h->device, h->staging_i, host, n * 4, h->stream));
+    HIPCHK(h, h->pipe.to_device(h->staging_i, host, n * 4, h->stream));
     k_i32_to_u8<<<grid_blocks(n), 256, 0, h->stream>>>(h->staging_i, h->ID, n, h->s.inactive, &h->cnt->inactive_seen,
                                                         ++h->id_uploads);
     if (!h->multimat) {
@@ -765,11 +766,11 @@ int m2cx_upload(m2cx_solver* h, int field, const void* host) {
     }
   } else if (field == M2CX_FIELD_PHI) {
     if (!h->mp.phi) return fail(h, M2CX_E_ARG, "no level set");
-    HIPCHK(h, h->pipe.to_device(h->device, h->mp.phi, host, n * 8, h->stream));
+    HIPCHK(h, h->pipe.to_device(h->mp.phi, host, n * 8, h->stream));
   } else {
     double** f = field_ptr(h, field);
     if (!f) return fail(h, M2CX_E_ARG, "bad field");
-    HIPCHK(h, h->pipe.to_device(h->device, h->staging, host, n * 5 * 8, h->stream));
+    HIPCHK(h, h->pipe.to_device(h->staging, host, n * 5 * 8, h->stream));
     k_aos_to_soa<<<grid_blocks(n), 256, 0, h->stream>>>(h->staging, f5(h, f), 5, n);
   }
   HIPCHK(h, hipGetLastError());
@@ -784,16 +785,16 @@ int m2cx_download(m2cx_solver* h, int field, void* host) {
   if (field == M2CX_FIELD_ID) {
     k_u8_to_i32<<<grid_blocks(n), 256, 0, h->stream>>>(h->ID, h->staging_i, n);
     HIPCHK(h, hipGetLastError());
-    HIPCHK(h, h->pipe.to_host(h->device, host, h->staging_i, n * 4, h->stream));
+    HIPCHK(h, h->pipe.to_host(host, h->staging_i, n * 4, h->stream));
   } else if (field == M2CX_FIELD_PHI) {
     if (!h->mp.phi) return fail(h, M2CX_E_ARG, "no level set");
-    HIPCHK(h, h->pipe.to_host(h->device, host, h->mp.phi, n * 8, h->stream));
+    HIPCHK(h, h->pipe.to_host(host, h->mp.phi, n * 8, h->stream));
   } else {
     double** f = field_ptr(h, field);
     if (!f) return fail(h, M2CX_E_ARG, "bad field");
     k_soa_to_aos<<<grid_blocks(n), 256, 0, h->stream>>>(cf5(h, f), h->staging, 5, n);
     HIPCHK(h, hipGetLastError());
-    HIPCHK(h, h->pipe.to_host(h->device, host, h->staging, n * 5 * 8, h->stream));
+    HIPCHK(h, h->pipe.to_host(host, h->staging, n * 5 * 8, h->stream));
   }
   return 0;
 }
@@ -2117,7 +2118,7 @@ int m2cx_levelset_residual(m2cx_solver* h, int v_field) {
 int m2cx_download_ls_residual(m2cx_solver* h, double* host) {
   if (!h || !h->mp.rls) return M2CX_E_ARG;
   HIPCHK(h, hipSetDevice(h->device));
-  HIPCHK(h, h->pipe.to_host(h->device, host, h->mp.rls, h->ncells * 8, h->stream));
+  HIPCHK(h, h->pipe.to_host(host, h->mp.rls, h->ncells * 8, h->stream));
   return 0;
 }
 

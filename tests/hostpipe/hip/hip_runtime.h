@@ -28,6 +28,7 @@ struct FakeHip {
   std::deque<Copy> todo;
   std::vector<Copy> log;
   size_t given = 0, done = 0;
+  size_t allocated = 0;  // calls of hipHostMalloc
   bool stop = false, no_pinned = false, unregistered_is_error = false;
   long fail_copy = -1;  // the copy with this number is refused
   std::map<const char*, size_t> pinned;
@@ -75,6 +76,7 @@ inline hipError_t hipGetLastError() { return hipSuccess; }
 inline hipError_t hipHostMalloc(void** p, size_t n, unsigned) {
   if (fake().no_pinned) return hipErrorOutOfMemory;
   *p = std::malloc(n);
+  { std::lock_guard<std::mutex> l(fake().mu); fake().allocated++; }
   fake().pin(*p, n);
   return hipSuccess;
 }

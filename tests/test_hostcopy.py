@@ -47,3 +47,14 @@ def test_a_failing_copy_is_reported(driver, way):
     first, second = driver("link-fails", way, 40 * MB)
     assert first[0] != 0 and first[2] == 5
     assert second[:3] == (0, 1, 20)
+
+
+def test_solvers_share_a_ring(driver):
+    """One after another they use the same one; it goes with the last of them."""
+    assert driver("solvers", "up", 9 * MB, 5) == [(0, 1, 1, 0)]
+
+
+def test_solvers_copying_at_once(driver):
+    """Each copy has a ring to itself, and at most two are kept."""
+    (bad, allocated, held, left), = driver("solvers", "down", 9 * MB, 5)
+    assert bad == 0 and 1 <= allocated <= 15 and 1 <= held <= 2 and left == 0
